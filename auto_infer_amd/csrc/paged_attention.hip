@@ -2187,9 +2187,13 @@ struct MergeArgs {
 // kFixParts), a compile-time count so that the loads are issued
 // unconditionally and the compiler's counter waits for the header words
 // leave them in flight.
-template <int kMergeGroups, int FIXL>
+// EL: elements per work-group, 64 (a record's slice) or 8 (an eighth of it:
+// one row at head_dim 128).  See launch_merge.
+template <int kMergeGroups, int FIXL, int EL>
 __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   constexpr int kMergeThreads = 64 * kMergeGroups;
+  constexpr int kSub = 64 / EL;                           // work-groups per record
+  static_assert(EL == 64 || (EL == 8 && FIXL == 0), "whole slices or eighths");
   constexpr int kLdsGroups = kMergeGroups > 1 ? kMergeGroups - 1 : 1;
   __shared__ float4 sacc[kLdsGroups][kMergeDims / 4][64];
   __shared__ float2 sml[kLdsGroups][64];
@@ -2217,7 +2221,8 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   int vz;
   asm volatile("v_mov_b32 %0, 0" : "=v"(vz));
   const int64_t item0 = blockIdx.x;
-  const int4* mp = (item0 < a.mrg_cap ? reinterpret_cast<const int4*>(a.mrg + item0 * kMrgInts)
+  const int64_t rec0 = item0 / kSub;
+  const int4* mp = (rec0 < a.mrg_cap ? reinterpret_cast<const int4*>(a.mrg + rec0 * kMrgInts)
                                       : reinterpret_cast<const int4*>(a.hdr)) + vz;
   const int4* pp0 = (a.pf_mrg && item0 < a.pf_items_cap ? a.pf_mrg + (int)blockIdx.x / per_rec
                                                           : reinterpret_cast<const int4*>(a.hdr)) + vz;
@@ -2360,22 +2365,25 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   }
   // the first test reads the first record too (a record has at least two
   // parts), which keeps its loads ahead of the first branch
-  const bool first_live = (fixed_plan != 1) & (item0 < a.mrg_cap) & (item0 < nmrg) &
+  const bool first_live = (fixed_plan != 1) & (rec0 < a.mrg_cap) & (rec0 < nmrg) &
                           (m1_first.y >= 2);
-  for (int64_t item = item0; first_live && item < a.mrg_cap; item += gridDim.x) {
-    if (item >= nmrg) break;                               // uniform over the group
-    const int4 m0 = item == item0 ? m0_first : *reinterpret_cast<const int4*>(a.mrg + item * kMrgInts);
-    const int4 m1 = item == item0 ? m1_first : *reinterpret_cast<const int4*>(a.mrg + item * kMrgInts + 4);
+  for (int64_t item = item0; first_live && item < a.mrg_cap * kSub; item += gridDim.x) {
+    const int64_t mrec = item / kSub;
+    if (mrec >= nmrg) break;                               // uniform over the group
+    const int4 m0 = item == item0 ? m0_first : *reinterpret_cast<const int4*>(a.mrg + mrec * kMrgInts);
+    const int4 m1 = item == item0 ? m1_first : *reinterpret_cast<const int4*>(a.mrg + mrec * kMrgInts + 4);
     const int qtok0 = m0.x, nq = m0.y, kvh = m0.z, hbi = m0.w;
     const int row_base = m1.x, np = m1.y, sl = m1.z, rows = m1.w;
     // A slice of fewer than 64 elements (a decode segment's few rows) takes
     // the smallest power-of-two lane group that holds it, and the wave's
     // other lane groups fold other partials: all of an item's partial loads
     // then go out in one round (config 1: 16 elements, 16 partials at once).
-    const int span = rows * epr - sl * 64;
-    const int pw = span > 32 ? 64 : span > 16 ? 32 : span > 8 ? 16 : 8;
+    const int e0 = sl * 64 + (int)(item - mrec * kSub) * EL;   // the work-group's first element
+    const int span = rows * epr - e0;
+    if (EL < 64 && span <= 0) continue;                    // past the slice's rows (uniform)
+    const int pw = EL < 64 ? EL : span > 32 ? 64 : span > 16 ? 32 : span > 8 ? 16 : 8;
     const int pg = lane / pw, ng = 64 / pw;
-    const int e = sl * 64 + (lane & (pw - 1));
+    const int e = e0 + (lane & (pw - 1));
     int n = e / epr;
     const int c = (e - n * epr) * kMergeDims;
     const int rblk = n / kRows, t = (n - rblk * kRows) / a.hb;
@@ -2391,7 +2399,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
     float mx = -1e30f, ls = 0.f;
     auto fold = [&](float2 ml, const float4 (&x)[kMergeDims / 4]) { fold_into(mx, ls, acc, ml, x); };
     if (live) {    // fp16 partials y = O / c, with (m + log2 c, l / c)
-#pragma unroll 2
+#pragma unroll(EL < 64 ? 4 : 2)
       for (int k = kg * ng + pg; k < np; k += kMergeGroups * ng) {
         const int64_t pr = row0 + k * pstride;
         const float2 ml = a.part_ml[pr];
@@ -3149,7 +3157,20 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   mg.pf_mrg = pf ? reinterpret_cast<const int4*>(ws + L.pfm) : nullptr;
   // wide: 64-element slices (MLA, or 8+ rows per segment) and about 8 or
   // more ranges per segment, i.e. a dozen partials per item
-  const bool wide = AIA_MERGE_WIDE && L.pf_mrg_cap == 0 &&
+  // deep: few segments over many ranges each (a handful of long requests).
+  // A record's 64 elements then go to eight work-groups, one row of head_dim
+  // 128 each, whose lane groups fold 32 parts at a time instead of 4 or 8:
+  // with whole slices a few work-groups walked hundreds of parts (one request
+  // of 32K keys, 28/4 heads: 512 parts on 4 work-groups, 57 us per call; 21.7
+  // with eighths.  16 latent heads, 32K keys: 54.9 -> 27.0).  At 64 ranges per
+  // segment eighths win everywhere (28/4 heads x 8 requests 37.2 -> 33.3, 64/8
+  // x 4 34.2 -> 32.0, 16/8 x 4 32.4 -> 31.4, 14/2 x 16 19.5 -> 17.5); at 32 they
+  // are between 34.6 -> 33.9 (28/4) and 48.7 -> 49.8 (16/8, whose whole slices
+  // have fixed slots), and at 16 52.1 -> 54.3: more work-groups than loads to
+  // spread.  (8 and 16 waves per work-group: slower.)
+  const int64_t blocks = std::max<int64_t>(batch, (tokens + g.qs - 1) / g.qs);
+  const bool deep = (int64_t)waves >= 64 * blocks * g.nkvg * g.nhb;
+  const bool wide = AIA_MERGE_WIDE && !deep && L.pf_mrg_cap == 0 &&
                     (dv == kMlaV || (int64_t)g.hb * ((tokens + batch - 1) / batch) >= 8) &&
                     (int64_t)waves >= 8LL * batch * g.nkvg * g.nhb;
   const int threads = wide ? 512 : 256;
@@ -3158,7 +3179,8 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   mg.pf_o = reinterpret_cast<const uint16_t*>(ws + L.pf_o);
   mg.pf_ml = reinterpret_cast<const float2*>(ws + L.pf_ml);
   const int64_t pitems = pf ? L.pf_mrg_cap * g.hkv * pf_slices : 0;
-  const int64_t items = L.mrg_cap > pitems ? L.mrg_cap : pitems;
+  const int64_t mitems = deep ? 8 * L.mrg_cap : L.mrg_cap;
+  const int64_t items = mitems > pitems ? mitems : pitems;
   int64_t mgrid = items < 2048 ? items : 2048;
   if (mgrid < 1) mgrid = 1;
   // Fixed-slot merges for small steps (kFixParts): one work-group per
@@ -3171,7 +3193,7 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   // loads per thread 40.6 -> 42 us, config 1 then 21.9 -> 22.75.)
   mg.fixed_slots = 0;
   mg.part_cap = L.part_cap;
-  if (small_geometry(g, dv, batch, L.seg_cap) && L.part_cap >= kFixParts * L.seg_cap) {
+  if (!deep && small_geometry(g, dv, batch, L.seg_cap) && L.part_cap >= kFixParts * L.seg_cap) {
     const int64_t nq_max = std::min<int64_t>(g.qs, (int64_t)tokens - batch + 1);
     const int64_t rows_max = std::min<int64_t>(
         (int64_t)kRows * g.rb, nq_max <= g.qb ? nq_max * g.hb : (int64_t)kRows * ((nq_max + g.qb - 1) / g.qb));
@@ -3183,11 +3205,12 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   if (mg.fixed_slots && !wide) {
     // kFixWaves waves of kFixParts / (4 kFixWaves) slot loads per thread (config 1,
     // us per layer: 2 waves 21.62-21.66, 1 wave 21.87-21.91, 4 waves 21.86-21.89)
-    merge_kernel<kFixWaves, kFixParts / (4 * kFixWaves)><<<(unsigned)mgrid, 64 * kFixWaves, 0, s>>>(mg);
+    merge_kernel<kFixWaves, kFixParts / (4 * kFixWaves), 64><<<(unsigned)mgrid, 64 * kFixWaves, 0, s>>>(mg);
     return aia::check_hip(hipGetLastError(), "merge_kernel launch");
   }
-  if (wide) merge_kernel<8, 0><<<(unsigned)mgrid, threads, 0, s>>>(mg);
-  else merge_kernel<4, 0><<<(unsigned)mgrid, threads, 0, s>>>(mg);
+  if (deep) merge_kernel<4, 0, 8><<<(unsigned)mgrid, threads, 0, s>>>(mg);
+  else if (wide) merge_kernel<8, 0, 64><<<(unsigned)mgrid, threads, 0, s>>>(mg);
+  else merge_kernel<4, 0, 64><<<(unsigned)mgrid, threads, 0, s>>>(mg);
   return aia::check_hip(hipGetLastError(), "merge_kernel launch");
 }
 

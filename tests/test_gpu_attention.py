@@ -519,3 +519,27 @@ def test_fixed_slot_merge_decode_steps(hq, hkv, waves):
     print(f"hq {hq} hkv {hkv} waves {waves}: header {hdr[:11].tolist()}, max-abs err {err:.3e}",
           flush=True)
     assert err <= TOL, err
+
+
+@pytest.mark.parametrize("hq,hkv,d,lqs,lks", [
+    (28, 4, 128, [1], [9000]),                    # one long request, 512 ranges
+    (7, 1, 128, [1], [5]),                        # a single range beside idle slots
+    (14, 2, 64, [1, 1, 1], [4000, 17, 1]),        # 4 elements a row: part-filled eighths
+    (40, 2, 128, [1, 3], [3000, 900]),            # a part-filled second head block
+    (32, 8, 128, [2, 1, 2], [2500, 2, 700]),      # verify rows, whole eighths past the rows
+])
+def test_few_long_requests_merge_in_eighths(hq, hkv, d, lqs, lks):
+    """Few segments over many ranges: eight work-groups per merge record.  A
+    sentinel in the output shows a row the merge misses or a stray write."""
+    step = workloads.make_gqa_step(lqs=lqs, lks=lks, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
+                                   block_size=16, seed=hq + d)
+    s = step
+    plan = ops.AttentionPlan.from_lists(s.block_table.to(DEV), s.cu_seqlens_q, s.seqlens_kv,
+                                        hq, hkv, d, 16)
+    out = torch.full(s.q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention_gqa(s.q.to(DEV), s.k_cache.to(DEV), s.v_cache.to(DEV), plan, s.scale,
+                            out=out)
+    torch.cuda.synchronize()
+    err = (out.float().cpu() - oracle(step)).abs().max().item()
+    print(f"max-abs err {err:.3e}", flush=True)
+    assert err <= TOL, err

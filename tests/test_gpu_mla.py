@@ -41,6 +41,13 @@ def test_mla_split_invariance(waves):
     check(step, waves)
 
 
+@pytest.mark.parametrize("lqs,lks,heads", [([1], [9000], 16), ([2, 1], [5000, 40], 16),
+                                           ([1, 1], [3000, 1], 20)])
+def test_mla_few_long_requests_merge_in_eighths(lqs, lks, heads):
+    """768 ranges over one or two requests: eight work-groups per merge record."""
+    check(workloads.make_mla_step(lqs=lqs, lks=lks, num_heads=heads, block_size=64, seed=heads))
+
+
 def test_mla_multi_token_query_causal():
     step = workloads.make_mla_step(lqs=[2, 3, 1], lks=[300, 40, 5], block_size=64, seed=6)
     check(step)

@@ -6,11 +6,11 @@
 // last step (new blocks, new tokens, drafts) and (b) one 8-int descriptor per
 // sequence row.  Two kernels then run:
 //   pack_updates  scatter of the changed pool entries;
-//   pack_rows     one wave per row: positions start..start+n-1, token ids
-//                 gathered from the token pool, slot = block[pos / bs] * bs +
-//                 pos % bs, the zero-padded block-table row, cu_seqlens_q,
-//                 seqlens_kv = start + n, the last-row index of every row and
-//                 the compacted sample rows.
+//   pack_rows     some waves per row (see kChunk): positions start..start+n-1,
+//                 token ids gathered from the token pool, slot =
+//                 block[pos / bs] * bs + pos % bs, the zero-padded block-table
+//                 row, cu_seqlens_q, seqlens_kv = start + n, the last-row index
+//                 of every row and the compacted sample rows.
 // Synthetic rows (the stagers' scratch padding) take consecutive blocks
 // block_base, block_base + 1, ... and token id 0.
 #include <string.h>
@@ -50,26 +50,59 @@ __global__ __launch_bounds__(256) void pack_updates_kernel(
   }
 }
 
-// One row's outputs, by one wave.
-__device__ __forceinline__ void pack_one_row(const PackArgs& a, int r, const int32_t* d, int lane) {
+// A row's tokens and block-table columns are cut into chunks of kChunk, chunk
+// k of every row to wave k of the row's `nchunks`.  Every wave is a chain of
+// dependent loads (descriptor, block id, store) whatever it moves, so its
+// length is what the kernel takes: one wave per row walked a 1991-column table
+// row, or a 1657-token prompt, 64 at a time (14-16 us; chunked, with a
+// chunk's loads issued before its stores, 3.6 us).
+constexpr int kChunk = 256;
+constexpr int kMaxChunks = 64;     // a longer row's chunks go round
+
+__device__ __forceinline__ void pack_one_row(const PackArgs& a, int r, const int32_t* d, int lane,
+                                             int chunk, int nchunks) {
+  constexpr int kPer = kChunk / 64;
   const int src = d[0], start = d[1], n = d[2], nblocks = d[3], base = d[4], q_off = d[5];
   const int zero_tokens = d[6], sample_slot = d[7];
   const int32_t* prow = src >= 0 ? a.block_pool + (int64_t)src * a.block_stride : nullptr;
   const int64_t* trow = src >= 0 ? a.token_pool + (int64_t)src * a.token_stride : nullptr;
   const int max_col = (int)a.block_stride - 1;
-  for (int j = lane; j < n; j += 64) {
-    const int pos = start + j;
-    const int bi = pos / a.block_size;
-    const int blk = prow ? prow[min(bi, max_col)] : base + bi;
-    const int64_t q = q_off + j;
-    a.positions[q] = pos;
-    a.slot_mapping[q] = blk * a.block_size + (pos - bi * a.block_size);
-    a.token_ids[q] = (zero_tokens || !trow) ? 0 : trow[min((int64_t)pos, a.token_stride - 1)];
+  for (int j0 = chunk * kChunk; j0 < n; j0 += nchunks * kChunk) {
+    int blk[kPer], off[kPer];
+    int64_t tok[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int j = min(j0 + 64 * i + lane, n - 1);
+      const int bi = (start + j) / a.block_size;
+      off[i] = start + j - bi * a.block_size;
+      blk[i] = prow ? prow[min(bi, max_col)] : base + bi;
+      tok[i] = (zero_tokens || !trow) ? 0 : trow[min((int64_t)(start + j), a.token_stride - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int j = j0 + 64 * i + lane;
+      if (j >= n) break;
+      const int64_t q = q_off + j;
+      a.positions[q] = start + j;
+      a.slot_mapping[q] = blk[i] * a.block_size + off[i];
+      a.token_ids[q] = tok[i];
+    }
   }
   int32_t* bt = a.block_table + (int64_t)r * a.bt_width;
-  for (int c = lane; c < a.bt_width; c += 64)
-    bt[c] = c < nblocks ? (prow ? prow[min(c, max_col)] : base + c) : 0;
-  if (lane == 0) {
+  for (int c0 = chunk * kChunk; c0 < a.bt_width; c0 += nchunks * kChunk) {
+    int v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = c0 + 64 * i + lane;
+      v[i] = c < nblocks ? (prow ? prow[min(c, max_col)] : base + c) : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = c0 + 64 * i + lane;
+      if (c < a.bt_width) bt[c] = v[i];
+    }
+  }
+  if (lane == 0 && chunk == 0) {
     if (r == 0) a.cu_seqlens_q[0] = 0;
     a.cu_seqlens_q[r + 1] = q_off + n;
     a.seqlens_kv[r] = start + n;
@@ -78,22 +111,25 @@ __device__ __forceinline__ void pack_one_row(const PackArgs& a, int r, const int
   }
 }
 
-__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs a) {
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs a, int nchunks) {
   const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   // zero the unused tail of the sample rows (prefill stager contract)
   for (int i = blockIdx.x * blockDim.x + threadIdx.x + a.sample_count; i < a.sample_cap;
        i += gridDim.x * blockDim.x)
     a.sample_rows[i] = 0;
+  const int r = w / nchunks;
   if (r >= a.num_rows) return;
-  pack_one_row(a, r, a.rows + (int64_t)r * 8, lane);
+  pack_one_row(a, r, a.rows + (int64_t)r * 8, lane, w - r * nchunks, nchunks);
 }
 
-// The whole step in one work-group, its updates and row descriptors carried
-// in the kernel arguments (the launch copies them; no staging copy): the
-// pool updates first, then, after a work-group barrier (one CU, so its
-// stores are visible to the whole group), one wave per row; 16 waves, so a
-// decode gear of up to 16 requests packs its rows in one pass.
+// A small step in one launch, its updates and row descriptors carried in the
+// kernel arguments (the launch copies them; no staging copy): the pool updates
+// first, then, after a work-group barrier, one wave per row chunk.  Every
+// work-group makes all the updates itself before it reads (the same values to
+// the same places, at most 192 of them), so none waits for another; a step of
+// up to 16 chunks is one work-group of 16 waves.  (64 rows of a latent gear in
+// one work-group took 11 us, four row passes of 16 waves; in four, 4.2.)
 template <int BYTES>
 struct InlineBlob {
   int64_t w[BYTES / 8];
@@ -105,7 +141,7 @@ constexpr int kInlineSmall = 1024;
 template <int BYTES>
 __global__ __launch_bounds__(1024) void pack_inline_kernel(PackArgs a, InlineBlob<BYTES> blob, int32_t nt,
                                                           int32_t nb, int64_t* token_pool,
-                                                          int32_t* block_pool) {
+                                                          int32_t* block_pool, int32_t nchunks) {
   const int64_t* tidx = blob.w;
   const int64_t* tval = blob.w + nt;
   const int64_t* bidx = blob.w + 2 * nt;
@@ -115,11 +151,14 @@ __global__ __launch_bounds__(1024) void pack_inline_kernel(PackArgs a, InlineBlo
     if (i < nt) token_pool[tidx[i]] = tval[i];
     else block_pool[bidx[i - nt]] = bval[i - nt];
   }
-  for (int i = threadIdx.x + a.sample_count; i < a.sample_cap; i += blockDim.x) a.sample_rows[i] = 0;
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x + a.sample_count; i < a.sample_cap; i += blockDim.x) a.sample_rows[i] = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  for (int r = threadIdx.x >> 6; r < a.num_rows; r += blockDim.x >> 6)
-    pack_one_row(a, r, rows + (int64_t)r * 8, lane);
+  const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+  const int r = w / nchunks;
+  if (r >= a.num_rows) return;
+  pack_one_row(a, r, rows + (int64_t)r * 8, lane, w - r * nchunks, nchunks);
 }
 
 // Token splice: target[pairs[i].row] = *pairs[i].source for every pair, one
@@ -191,8 +230,12 @@ extern "C" int aia_pack_rows(const int64_t* token_update_index, const int64_t* t
   a.block_table = block_table; a.cu_seqlens_q = cu_seqlens_q; a.seqlens_kv = seqlens_kv;
   a.last_rows = last_rows; a.sample_rows = sample_rows;
   a.sample_count = sample_count; a.sample_cap = sample_cap;
-  const int grid = num_rows > 0 ? (num_rows + 3) / 4 : 1;
-  pack_rows_kernel<<<grid, 256, 0, s>>>(a);
+  // The rows are on the device, so their token counts are not known here: the
+  // table's width gives the chunks, and at least four for a prompt's tokens.
+  int nchunks = (block_table_width + kChunk - 1) / kChunk;
+  nchunks = nchunks < 4 ? 4 : nchunks > kMaxChunks ? kMaxChunks : nchunks;
+  const int64_t waves = (int64_t)num_rows * nchunks;
+  pack_rows_kernel<<<waves > 0 ? (unsigned)((waves + 3) / 4) : 1, 256, 0, s>>>(a, nchunks);
   return check_hip(hipGetLastError(), "pack_rows launch");
 }
 
@@ -231,17 +274,23 @@ extern "C" int aia_pack_rows_inline(const void* blob, int32_t num_token_updates,
   a.block_table = block_table; a.cu_seqlens_q = cu_seqlens_q; a.seqlens_kv = seqlens_kv;
   a.last_rows = last_rows; a.sample_rows = sample_rows;
   a.sample_count = sample_count; a.sample_cap = sample_cap;
+  // chunks per row from the longest row and the table's width
+  const int32_t* rows = static_cast<const int32_t*>(blob) + 2 * (2 * nt + nb + (nb + 1) / 2);
+  int32_t longest = nr > 0 ? block_table_width : 1;
+  for (int64_t r = 0; r < nr; ++r) longest = rows[8 * r + 2] > longest ? rows[8 * r + 2] : longest;
+  int32_t nchunks = (longest + kChunk - 1) / kChunk;
+  nchunks = nchunks < 1 ? 1 : nchunks > kMaxChunks ? kMaxChunks : nchunks;
+  const unsigned grid = nr > 0 ? (unsigned)((nr * nchunks + 15) / 16) : 1;
   if (words * 8 <= kInlineSmall) {
     InlineBlob<kInlineSmall> b;
     memcpy(b.w, blob, (size_t)words * 8);
-    pack_inline_kernel<kInlineSmall><<<1, 1024, 0, (hipStream_t)stream>>>(a, b, (int32_t)nt,
-                                                                          (int32_t)nb, token_pool,
-                                                                          block_pool);
+    pack_inline_kernel<kInlineSmall><<<grid, 1024, 0, (hipStream_t)stream>>>(
+        a, b, (int32_t)nt, (int32_t)nb, token_pool, block_pool, nchunks);
   } else {
     InlineBlob<AIA_PACK_INLINE_BYTES> b;
     memcpy(b.w, blob, (size_t)words * 8);
-    pack_inline_kernel<AIA_PACK_INLINE_BYTES><<<1, 1024, 0, (hipStream_t)stream>>>(
-        a, b, (int32_t)nt, (int32_t)nb, token_pool, block_pool);
+    pack_inline_kernel<AIA_PACK_INLINE_BYTES><<<grid, 1024, 0, (hipStream_t)stream>>>(
+        a, b, (int32_t)nt, (int32_t)nb, token_pool, block_pool, nchunks);
   }
   return check_hip(hipGetLastError(), "aia_pack_rows_inline launch");
 }

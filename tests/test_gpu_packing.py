@@ -252,3 +252,27 @@ def test_build_of_each_inline_argument_size(batch):
             views[rid] = RequestView(rid, tuple(range(100 + i, 100 + i + lk)), lk - 1, 1, 1, ())
             sched.append(ScheduledRequest(rid, 1, False, tables[rid]))
         check_build(packer, BatchPlan.make(sched, views, tables), bs)
+
+
+@pytest.mark.parametrize("inline", [True, False])
+@pytest.mark.parametrize("bs,chunks", [
+    (1, [(0, 255), (3, 256), (0, 257), (900, 1)]),       # tables and prompts at a chunk's edges
+    (16, [(0, 1657), (31000, 1), (5, 64)]),              # a long table beside a long prompt
+    (1, [(0, 16500), (16700, 1)]),                       # more than 64 chunks: they go round
+])
+def test_build_rows_cut_into_chunks(bs, chunks, inline, monkeypatch):
+    """Rows whose tokens and table columns span several waves' chunks; the
+    second build of a step has no updates and goes out inline."""
+    monkeypatch.setattr(packing, "_USE_INLINE", inline)
+    reqs, free = {}, iter(range(100000))
+    for i, (start, n) in enumerate(chunks):
+        reqs[f"r{i}"] = dict(tokens=[(7 * i + 3 * t) % 50000 for t in range(start + n)],
+                             computed=start, prompt=start + n, prefill=start + n, draft=[],
+                             blocks=[next(free) for _ in range((start + n + bs - 1) // bs)])
+    plan = make_plan(reqs, [(f"r{i}", n, n > 1) for i, (_, n) in enumerate(chunks)])
+    packer = packing.DeviceBatchPacker(bs, DEV)
+    for _ in range(2):
+        check_build(packer, plan, bs)
+        for t in (packer.token_ids_buf, packer.positions_buf, packer.slot_mapping_buf,
+                  packer.block_table_buf):
+            t.fill_(-1)

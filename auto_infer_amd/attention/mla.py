@@ -53,8 +53,7 @@ class MlaHipBackend(AttentionBackend):
         # With fuse_pre_attention, q_latent and k_latent each come from one
         # kernel (norm / interleave / RoPE / W_UK product / cat; bf16 rounding
         # where the torch ops round) when the shapes allow it (nope 128), and
-        # the W_UV product after attention from a third (v_head_dim 128, up to
-        # ops.MLA_V_UP_MAX_ROWS query rows; longer steps use the library GEMM).
+        # the W_UV product after attention from a third (v_head_dim 128).
         self.fuse_pre_attention = fuse_pre_attention
 
     def alloc_kv_caches(self, num_blocks: int, block_size: int) -> list:
@@ -123,7 +122,7 @@ class MlaHipBackend(AttentionBackend):
             k_latent = torch.cat([ckv.unsqueeze(1), k_pe], dim=-1).contiguous()
         self._write_kv(layer_idx, k_latent, None, ctx)
         o_latent = self._attn(layer_idx, q_latent, k_latent, None, ctx)
-        if fused and vd == 128 and T * nh <= ops.MLA_V_UP_MAX_ROWS:
+        if fused and vd == 128:
             o = ops.mla_v_up(o_latent, w_uv)
         else:
             o = torch.einsum("tnl,nvl->tnv", o_latent, w_uv)

@@ -51,7 +51,34 @@ __device__ __forceinline__ float group4_sum(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// One 16-byte direct load from global memory into LDS at byte lds + 16 lane
+// (lds wave-uniform).  Issued as inline assembly on purpose: the compiler's
+// counter-wait pass tracks the builtin form as an outstanding LDS access and
+// then waits for the LDS counter to drain completely (lgkmcnt(0)) before
+// every LDS read, which exposes each read's full latency (48.2 against 49.3
+// µs per call, and it defeats the read-ahead order above: 47.6-47.9 against
+// 46.0).  Completion is explicit instead: every step waits vmcnt(0) before its
+// barrier.  Loads the compiler does not see can only make its own vmcnt waits
+// stricter, never too weak (the counter retires in order).
+// m0 (the LDS address of the load) is named as clobbered, which clang warns
+// about for a register it reserves: the warning is silenced here because the
+// clobber is what tells the compiler that m0 changed, and the compiler keeps
+// no value of its own in m0 in these kernels (their device assembly sets m0
+// only in front of these loads).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_load16(const uint16_t* src, uint16_t* lds) {
+  const uint32_t la = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(la), "v"(src) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+
+// s_waitcnt vmcnt(0) (expcnt / lgkmcnt left at their maxima), gfx9 encoding:
+// what a lds_load16 needs before the barrier that publishes its bytes.
+constexpr int kWaitVmcnt0 = 0x0F70;
 
 }  // namespace aia

@@ -130,6 +130,11 @@ __device__ __forceinline__ bf16x8_t as_b8(uint4 v) {
   return __builtin_bit_cast(bf16x8_t, u32x4_t{v.x, v.y, v.z, v.w});
 }
 
+__device__ __forceinline__ uint4 pack8(aia::float4_t lo, aia::float4_t hi) {
+  return make_uint4(aia::pack_bf16x2(lo[0], lo[1]), aia::pack_bf16x2(lo[2], lo[3]),
+                    aia::pack_bf16x2(hi[0], hi[1]), aia::pack_bf16x2(hi[2], hi[3]));
+}
+
 // One work-group per (16 tokens, head, quarter of the latent).  q_latent^T
 // (latent x tokens) = W_UK^T (latent x 128) . q_nope^T (128 x tokens) on
 // v_mfma_f32_16x16x32_bf16: lane (latent m, group g) loads W_UK^T[h][m][32 j +
@@ -173,6 +178,77 @@ __global__ __launch_bounds__(256) void mla_q_latent_kernel(QArgs a) {
               a.out + (int64_t)tt * a.out_ts + (int64_t)h * a.out_hs + kLatent, k);
 }
 
+// Long steps (prefill): a work-group per (128 tokens, head, quarter of the
+// latent), wave w its tokens 32 w .. 32 w + 31 against all 128 latent columns
+// of the quarter.  The quarter of W_UK^T (32 KB, contiguous) goes straight into
+// LDS once and serves the four waves; read from global by every wave for its
+// own 16 tokens, as the decode kernel does, the L1 reads of W_UK bound the
+// kernel (2450 tokens x 16 heads, 45 MB written: 58.1 -> 17.7 us; with 32
+// tokens per wave and no LDS 28.9).
+//   Two 16-column MFMA tiles share 32 columns: row m of tile c holds column
+// 8 (m / 4) + 4 c + m % 4 of them, so a lane ends with 8 consecutive columns,
+// one 16-byte store.  LDS chunk c (16 bytes) of column r sits at c ^ f(r), f
+// distinct over a fragment read's 16 columns.  Work-group z rotates the pe part
+// of tokens 32 z .. 32 z + 31.
+constexpr int kQLongTokens = 128;
+__global__ __launch_bounds__(256) void mla_q_latent_long_kernel(QArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t wl[128 * kNope];
+  const int h = blockIdx.y, z = blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int tg = blockIdx.x * kQLongTokens, t0 = tg + 32 * wid;
+  auto swz = [](int r) { return (r & 3) | (((r >> 3) & 3) << 2); };
+  const uint16_t* wz = a.wukt + ((int64_t)h * kLatent + 128 * z) * kNope;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {      // 4 columns of 256 bytes per load
+    const int r0 = 32 * wid + 4 * i, r = r0 + (lane >> 4);
+    aia::lds_load16(wz + r * kNope + 8 * ((lane & 15) ^ swz(r)), wl + r0 * kNope);
+  }
+  uint4 bq[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int tb = min(t0 + 16 * i + n, a.tokens - 1);    // rows past the end are not stored
+    const uint16_t* qrow = a.q + (int64_t)tb * a.q_ts + (int64_t)h * a.q_hs + 8 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bq[i][j] = *reinterpret_cast<const uint4*>(qrow + 32 * j);
+  }
+  __builtin_amdgcn_s_waitcnt(aia::kWaitVmcnt0);
+  __syncthreads();
+#pragma unroll
+  for (int l0 = 0; l0 < 128; l0 += 32) {
+    uint4 aw[2][4];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int r = l0 + 8 * (n >> 2) + 4 * c + (n & 3);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        aw[c][j] = *reinterpret_cast<const uint4*>(wl + r * kNope + 8 * ((4 * j + g) ^ swz(r)));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      aia::float4_t acc[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        acc[c] = aia::float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_b8(aw[c][j]), as_b8(bq[i][j]), acc[c], 0, 0, 0);
+      }
+      const int t = t0 + 16 * i + n;
+      if (t < a.tokens)
+        *reinterpret_cast<uint4*>(a.out + (int64_t)t * a.out_ts + (int64_t)h * a.out_hs + 128 * z + l0 + 8 * g) =
+            pack8(acc[0], acc[1]);
+    }
+  }
+  const int tt = tg + 32 * z + (threadIdx.x >> 3), k = threadIdx.x & 7;
+  if (tt < a.tokens)
+    rope_lane(a.q + (int64_t)tt * a.q_ts + (int64_t)h * a.q_hs + kNope,
+              a.cos + (int64_t)tt * a.cos_ts, a.sin + (int64_t)tt * a.sin_ts,
+              a.out + (int64_t)tt * a.out_ts + (int64_t)h * a.out_hs + kLatent, k);
+}
+static_assert(kQLongTokens == 32 * (kLatent / 128), "a quarter's work-group rotates its 32 tokens");
+
 struct UvArgs {
   const uint16_t* o;        // o_latent rows (T, H, >= 512), strides o_ts / o_hs
   int64_t o_ts, o_hs;
@@ -192,7 +268,8 @@ struct UvArgs {
 // latent dims 128 w .. 128 w + 127 and wave 0 adds the four slices through
 // LDS, so every wave is short and a 64-token decode batch spreads over 256
 // work-groups.  Each work-group reads its 32 KB of W_UV, so the W_UV reads
-// grow with the token count: the kernel is for decode and verify batches.
+// grow with the token count: the kernel is for decode and verify batches, and
+// mla_v_up_long_kernel for longer steps.
 __global__ __launch_bounds__(256) void mla_v_up_kernel(UvArgs a) {
   constexpr int KS = 4, kSteps = kLatent / 32 / KS;
   __shared__ aia::float4_t red[KS - 1][2][64];
@@ -239,6 +316,94 @@ __global__ __launch_bounds__(256) void mla_v_up_kernel(UvArgs a) {
         make_uint2(aia::pack_bf16x2(acc0[0], acc0[1]), aia::pack_bf16x2(acc0[2], acc0[3]));
     *reinterpret_cast<uint2*>(dst + 16) =
         make_uint2(aia::pack_bf16x2(acc1[0], acc1[1]), aia::pack_bf16x2(acc1[2], acc1[3]));
+  }
+}
+
+// Long steps: a work-group per (64 tokens, head); wave (i, j) of 2 x 2 sums
+// tokens 32 i .. + 31 by v columns 64 j .. + 63.  The latent is walked 64 dims
+// at a time, both operands' slices (128 columns and 64 tokens of 128 bytes, 24
+// KB) loaded straight into one of two LDS buffers a slice ahead, so W_UV is
+// read once per 64 tokens and o_latent once (2450 tokens x 16 heads, 40 MB of
+// o_latent: 55.3 -> 12.9 us; library product 23.5).  Columns are dealt to MFMA
+// rows as in mla_q_latent_long_kernel, for 16-byte stores; LDS chunk c of row
+// r sits at c ^ f(r), f distinct over the eight rows of a fragment read's
+// cycle.
+constexpr int kUvLongTokens = 64;
+constexpr int kUvSlice = 64;                  // latent dims per LDS slice
+__global__ __launch_bounds__(256) void mla_v_up_long_kernel(UvArgs a) {
+  constexpr int kRows = kNope + kUvLongTokens;            // W_UV columns, then tokens
+  __shared__ __attribute__((aligned(16))) uint16_t buf0[kRows * kUvSlice];
+  __shared__ __attribute__((aligned(16))) uint16_t buf1[kRows * kUvSlice];
+  const int h = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int tg = blockIdx.x * kUvLongTokens;
+  const int tw = 32 * (wid >> 1), vw = 64 * (wid & 1);
+  auto wswz = [](int r) { return (r & 3) | (((r >> 3) & 1) << 2); };
+  // this lane's sources: 8 rows of 128 bytes per load, four loads of W_UV
+  // columns and two of tokens per wave
+  const int lr = lane >> 3, lc = lane & 7;
+  const uint16_t* src[6];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 32 * wid + 8 * i + lr;
+    src[i] = a.w + ((int64_t)h * kNope + r) * kLatent + 8 * (lc ^ wswz(r));
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 16 * wid + 8 * i + lr;
+    const int tb = min(tg + r, a.tokens - 1);             // rows past the end are not stored
+    src[4 + i] = a.o + (int64_t)tb * a.o_ts + (int64_t)h * a.o_hs + 8 * (lc ^ (r & 7));
+  }
+  auto load = [&](int s, uint16_t* buf) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      const int r0 = i < 4 ? 32 * wid + 8 * i : kNope + 16 * wid + 8 * (i - 4);
+      aia::lds_load16(src[i] + kUvSlice * s, buf + r0 * kUvSlice);
+    }
+  };
+  aia::float4_t acc[4][2];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[c][i] = aia::float4_t{0.f, 0.f, 0.f, 0.f};
+  auto slice = [&](const uint16_t* buf) {
+#pragma unroll
+    for (int j = 0; j < kUvSlice / 32; ++j) {
+      uint4 w[4], b[2];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int r = vw + 32 * (c >> 1) + 8 * (n >> 2) + 4 * (c & 1) + (n & 3);
+        w[c] = *reinterpret_cast<const uint4*>(buf + r * kUvSlice + 8 * ((4 * j + g) ^ wswz(r)));
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = tw + 16 * i + n;
+        b[i] = *reinterpret_cast<const uint4*>(buf + (kNope + r) * kUvSlice + 8 * ((4 * j + g) ^ (r & 7)));
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[c][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_b8(w[c]), as_b8(b[i]), acc[c][i], 0, 0, 0);
+    }
+  };
+  load(0, buf0);
+#pragma unroll
+  for (int s = 0; s < kLatent / kUvSlice; ++s) {
+    __builtin_amdgcn_s_waitcnt(aia::kWaitVmcnt0);
+    __syncthreads();          // slice s has arrived; slice s - 1 has been read
+    if (s + 1 < kLatent / kUvSlice) load(s + 1, s & 1 ? buf0 : buf1);
+    slice(s & 1 ? buf1 : buf0);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = tg + tw + 16 * i + n;
+    if (t >= a.tokens) continue;
+    uint16_t* dst = a.out + (int64_t)t * a.out_ts + (int64_t)h * a.out_hs + vw + 8 * g;
+    *reinterpret_cast<uint4*>(dst) = pack8(acc[0][i], acc[1][i]);
+    *reinterpret_cast<uint4*>(dst + 32) = pack8(acc[2][i], acc[3][i]);
   }
 }
 
@@ -296,6 +461,18 @@ extern "C" int aia_mla_q_latent(const void* q, int64_t q_token_stride, int64_t q
   a.cos_ts = cos_token_stride; a.sin_ts = sin_token_stride;
   a.out = static_cast<uint16_t*>(out); a.out_ts = out_token_stride; a.out_hs = out_head_stride;
   a.tokens = num_tokens; a.heads = num_heads;
+  // The 16-token kernel is the faster one while its work-groups fit one per
+  // CU (16 heads x 64 tokens, 256 work-groups: 3.89 against 4.20 us; 8 x 128
+  // 3.88 against 4.61), the 128-token one past that (16 x 96 5.14 against 4.46;
+  // 32 x 48 5.16 against 4.17; 128 x 8 4.95 against 4.63) if its 16-byte stores
+  // are aligned.
+  const int64_t tiles = ((int64_t)num_tokens + 15) / 16 * num_heads;
+  if (tiles > 64 && al16(out) && out_token_stride % 8 == 0 && out_head_stride % 8 == 0) {
+    const dim3 grid((unsigned)((num_tokens + kQLongTokens - 1) / kQLongTokens), (unsigned)num_heads,
+                    kLatent / 128);
+    mla_q_latent_long_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(a);
+    return check_hip(hipGetLastError(), "mla_q_latent_long launch");
+  }
   const dim3 grid((unsigned)((num_tokens + 15) / 16), (unsigned)num_heads, kLatent / 128);
   mla_q_latent_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(a);
   return check_hip(hipGetLastError(), "mla_q_latent launch");
@@ -320,6 +497,17 @@ extern "C" int aia_mla_v_up(const void* o_latent, int64_t o_token_stride, int64_
   a.w = static_cast<const uint16_t*>(w_uv);
   a.out = static_cast<uint16_t*>(out); a.out_ts = out_token_stride; a.out_hs = out_head_stride;
   a.tokens = num_tokens;
+  // The 16-token kernel up to two work-groups per CU (16 heads x 64 tokens
+  // 3.68 against 4.84 us, 32 x 32 3.66 against 4.68, 128 x 16, 512 work-groups,
+  // 5.08 against 6.39, 16 x 128 4.91 against 4.85), the 64-token one past that
+  // (16 x 192 6.20 against 4.94, 32 x 96 6.46 against 4.85, 128 x 32 8.06
+  // against 6.76) if its 16-byte stores are aligned.
+  const int64_t tiles = ((int64_t)num_tokens + 15) / 16 * num_heads;
+  if (tiles > 128 && al16(out) && out_token_stride % 8 == 0 && out_head_stride % 8 == 0) {
+    mla_v_up_long_kernel<<<dim3((unsigned)((num_tokens + kUvLongTokens - 1) / kUvLongTokens),
+                                (unsigned)num_heads), 256, 0, (hipStream_t)stream>>>(a);
+    return check_hip(hipGetLastError(), "mla_v_up_long launch");
+  }
   mla_v_up_kernel<<<dim3((unsigned)((num_tokens + 15) / 16), (unsigned)num_heads, 4), 256, 0,
                      (hipStream_t)stream>>>(a);
   return check_hip(hipGetLastError(), "mla_v_up launch");

@@ -1189,8 +1189,7 @@ __device__ __forceinline__ bool rec_ok(const int* r, int nseg_tiles, int batch, 
          r[6] <= nseg_tiles;
 }
 
-// s_waitcnt vmcnt(0) (expcnt / lgkmcnt left at their maxima), gfx9 encoding.
-constexpr int kWaitVmcnt0 = 0x0F70;
+using aia::kWaitVmcnt0;
 
 __device__ __forceinline__ short4_t as_s4(uint32_t a, uint32_t b) {
   short4_t r;
@@ -1616,28 +1615,6 @@ constexpr int kKStride = kHeadDim;   // the mixed kernel's (D = 128) buffer rows
 constexpr int kPfQkAhead = 2;
 constexpr int kPfPvAhead = 4;
 constexpr int kSgMfma = 0x008, kSgDsRead = 0x100;    // sched_group_barrier masks
-// One 16-byte direct load from global memory into LDS at byte lds + 16 lane
-// (lds wave-uniform).  Issued as inline assembly on purpose: the compiler's
-// counter-wait pass tracks the builtin form as an outstanding LDS access and
-// then waits for the LDS counter to drain completely (lgkmcnt(0)) before
-// every LDS read, which exposes each read's full latency (48.2 against 49.3
-// µs per call, and it defeats the read-ahead order above: 47.6-47.9 against
-// 46.0).  Completion is explicit instead: every step waits vmcnt(0) before its
-// barrier.  Loads the compiler does not see can only make its own vmcnt waits
-// stricter, never too weak (the counter retires in order).
-// m0 (the LDS address of the load) is named as clobbered, which clang warns
-// about for a register it reserves: the warning is silenced here because the
-// clobber is what tells the compiler that m0 changed, and the compiler keeps
-// no value of its own in m0 in these kernels (their device assembly sets m0
-// only in front of these loads).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_load16(const uint16_t* src, uint16_t* lds) {
-  const uint32_t la = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(la), "v"(src) : "memory", "m0");
-}
-#pragma clang diagnostic pop
 constexpr float kLazyLog2 = AIA_PF_LAZY;              // max growth (log2) before a rescale
 
 // Prefill attention: one work-group per (prefill item, kv head).  An item is
@@ -1841,8 +1818,8 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
       vp = fresh ? vnb + tok * a.vn_ts + 8 * cv : vp;
     }
     const int rb = (kLdKeys * i + kWaveKeys * wid) * D;     // the wave's first row
-    lds_load16(kp, kdst + rb);
-    lds_load16(vp, vdst + rb);
+    aia::lds_load16(kp, kdst + rb);
+    aia::lds_load16(vp, vdst + rb);
   };
   auto load = [&](int t, auto buf_tag) {
     constexpr int B = decltype(buf_tag)::value;
@@ -2941,10 +2918,10 @@ void mla_prefill_kernel(PrefillArgs a) {
     for (int i = 0; i < kMlaSub / kPfWaves; ++i) {
       const int r = wid * (kMlaSub / kPfWaves) + i;
       const int slot = __builtin_amdgcn_readfirstlane(sl[r]);
-      lds_load16(a.kc + (int64_t)slot * kMlaK + 8 * lane, dst + r * kMlaPfRow);
+      aia::lds_load16(a.kc + (int64_t)slot * kMlaK + 8 * lane, dst + r * kMlaPfRow);
     }
     const int r = wid * (kMlaSub / kPfWaves) + (lane >> 3);
-    lds_load16(a.kc + (int64_t)sl[r] * kMlaK + kMlaV + 8 * ((lane & 7) ^ (r & 7)),
+    aia::lds_load16(a.kc + (int64_t)sl[r] * kMlaK + kMlaV + 8 * ((lane & 7) ^ (r & 7)),
                dst + kMlaPfRope + wid * (kMlaSub / kPfWaves) * 64);
   };
 

@@ -136,20 +136,11 @@ def mla_q_latent(q, w_uk_t, cos, sin, out=None):
     return out
 
 
-# Query rows (tokens x heads) up to which mla_v_up beats the library GEMM
-# (measured at 16 heads: 7.3 against 11.3 us at 256 tokens; from 320 tokens
-# the library switches algorithm and wins, 6.9 against 8.6 us).
-MLA_V_UP_MAX_ROWS = 4096
-
-
 def mla_v_up(o_latent, w_uv, out=None):
     """Absorbed-MLA value up-projection, one launch: ``einsum("tnl,nvl->tnv",
     o_latent[..., :512], W_UV)`` (auto_infer/layers/attention/mla.py:120-121)
     for ``o_latent`` (T, H, >= 512) and ``w_uv`` (H, 128, 512) contiguous.
-    Returns ``out`` (T, H, 128); its (T, H * 128) view feeds o_proj.  Every
-    16-token work-group reads its share of W_UV, so the kernel is for decode
-    and verify batches (up to ``MLA_V_UP_MAX_ROWS`` rows); it is correct at
-    any size."""
+    Returns ``out`` (T, H, 128); its (T, H * 128) view feeds o_proj."""
     _check_device_tensor(o_latent, "o_latent", _BF16)
     _require(o_latent.dim() == 3 and o_latent.shape[2] >= MLA_LATENT and o_latent.stride(2) == 1,
              "o_latent must be (T, H, >= 512) with unit inner stride")

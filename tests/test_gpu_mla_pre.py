@@ -42,7 +42,8 @@ def close_to_one_ulp(got, exp, row_relative):
     assert same >= 0.99
 
 
-@pytest.mark.parametrize("T,H", [(1, 16), (7, 16), (64, 16), (33, 128), (300, 4)])
+@pytest.mark.parametrize("T,H", [(1, 16), (7, 16), (64, 16), (33, 128), (300, 4),
+                                 (65, 16), (127, 16), (129, 16), (1031, 1), (700, 20)])
 def test_q_latent_vs_oracle(T, H):
     q, w_uk, _, _, cos, sin = case(T, H, seed=T + H)
     got = ops.mla_q_latent(q.to(DEV), w_uk.transpose(1, 2).contiguous().to(DEV), cos.to(DEV),
@@ -96,10 +97,9 @@ def test_rejects_bad_shapes():
 
 
 @pytest.mark.parametrize("T,H", [(1, 16), (7, 16), (64, 16), (65, 16), (300, 4), (200, 128),
-                                 (2049, 16)])
+                                 (2049, 16), (129, 16), (145, 16), (2113, 1), (17, 65)])
 def test_v_up_vs_oracle(T, H):
-    """Decode / verify sizes and, beyond the rows the backend routes to it,
-    long steps, with ragged last token tiles."""
+    """Decode / verify sizes and long steps, with ragged last token tiles."""
     g = torch.Generator().manual_seed(T * 7 + H)
     o = (torch.randn(T, H, 512, generator=g) / 4).bfloat16()
     w_uv = (torch.randn(H, 128, 512, generator=g) / 11).bfloat16()
@@ -118,6 +118,27 @@ def test_v_up_strided_views():
     ops.mla_v_up(wide, w_uv, out=flat.view(T, H, 128))
     dense = ops.mla_v_up(wide[..., :512].contiguous(), w_uv)
     assert torch.equal(flat.view(T, H, 128), dense)
+
+
+@pytest.mark.parametrize("T,H", [(700, 20), (9, 8)])
+def test_latents_into_strided_outputs(T, H):
+    """Outputs as views of wider rows: 16-byte aligned ones take either
+    kernel's route, 8-byte aligned ones the 16-token kernels'.  The routes add
+    the fp32 products in other orders and round once, so they agree within
+    one bf16 ulp; nothing is written beside the views."""
+    q, w_uk, _, _, cos, sin = case(T, H, seed=T)
+    g = torch.Generator().manual_seed(T)
+    o = (torch.randn(T, H, 512, generator=g) / 4).bfloat16().to(DEV)
+    w_uv = (torch.randn(H, 128, 512, generator=g) / 11).bfloat16().to(DEV)
+    wt, q, cos, sin = w_uk.transpose(1, 2).contiguous().to(DEV), q.to(DEV), cos.to(DEV), sin.to(DEV)
+    for width, fn in ((576, lambda out: ops.mla_q_latent(q, wt, cos, sin, out=out)),
+                      (128, lambda out: ops.mla_v_up(o, w_uv, out=out))):
+        dense = fn(torch.empty(T, H, width, dtype=torch.bfloat16, device=DEV))
+        for lo, pad in ((8, 16), (4, 12), (0, 4)):
+            wide = torch.full((T, H, width + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+            fn(wide[..., lo:lo + width])
+            close_to_one_ulp(wide[..., lo:lo + width].cpu(), dense.cpu(), row_relative=False)
+            assert bool((wide[..., :lo] == 7).all()) and bool((wide[..., lo + width:] == 7).all())
 
 
 def test_v_up_rejects_bad_shapes():

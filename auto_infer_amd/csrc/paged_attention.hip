@@ -2170,6 +2170,7 @@ template <int kMergeGroups, int FIXL, int EL>
 __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   constexpr int kMergeThreads = 64 * kMergeGroups;
   constexpr int kSub = 64 / EL;                           // work-groups per record
+  constexpr int kUnroll = EL < 64 ? 4 : 2;                // parts whose loads go out together
   static_assert(EL == 64 || (EL == 8 && FIXL == 0), "whole slices or eighths");
   constexpr int kLdsGroups = kMergeGroups > 1 ? kMergeGroups - 1 : 1;
   __shared__ float4 sacc[kLdsGroups][kMergeDims / 4][64];
@@ -2376,7 +2377,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
     float mx = -1e30f, ls = 0.f;
     auto fold = [&](float2 ml, const float4 (&x)[kMergeDims / 4]) { fold_into(mx, ls, acc, ml, x); };
     if (live) {    // fp16 partials y = O / c, with (m + log2 c, l / c)
-#pragma unroll(EL < 64 ? 4 : 2)
+#pragma unroll kUnroll
       for (int k = kg * ng + pg; k < np; k += kMergeGroups * ng) {
         const int64_t pr = row0 + k * pstride;
         const float2 ml = a.part_ml[pr];
@@ -2807,48 +2808,82 @@ void mla_attn_kernel(MlaArgs a) {
 // its first 512, Hq query heads), planned as the GQA units are (128-row items
 // of one request's (token, head) rows, cut into key chunks when they are
 // few, chunk partials folded by the merge kernel).  A work-group of 4 waves,
-// one per SIMD, takes its unit's rows in two passes of 64, 16 rows per wave:
-//   Q (16 rows x 576) as MFMA operands in registers (72 VGPRs) and O (16 x
-//   512 fp32, 128 registers); 32 rows per wave would need about 400;
-//   keys go through LDS in 32-key sub-tiles, a ring of four buffers filled by
-//   direct loads three sub-tiles ahead (at one wave per SIMD no other wave
-//   covers a load's latency), one barrier per sub-tile;
-//   per sub-tile: QK^T over 576 dims (four accumulation chains per 16 keys),
-//   softmax, PV over the first 512 dims (V^T through transposing reads).
-// The cache slots of a sub-tile's keys are computed by wave 0 four
-// sub-tiles ahead from the unit's block ids, which it stages in LDS (2048
-// at a time) so that no load the compiler tracks sits behind the direct
-// loads in the loop (its wait would drain them).
-// LDS sub-tile: the 512 latent values of key r (1 KB, one direct load) at
-// row r of stride 1040 bytes -- the 16-byte pad puts the 16 keys of a K
-// fragment read, and the keys of a V^T read group, on different banks --
-// then the 64 rope values of every key, 128 bytes per key, its eight 16-byte
-// chunks swizzled (chunk c at c ^ (r mod 8)) since eight keys' rope share
-// one direct load.
+// one per SIMD, takes its unit's 128 rows together, on 32x32x16 MFMA:
+//   QK^T and softmax: wave w the 32 rows 32 w .. over all 576 dims, Q^T
+//   fragments in registers (144);
+//   PV: wave w the output dims 128 w .. + 127 of all 128 rows, O^T in the
+//   accumulation registers (256), so a V^T fragment read from LDS serves
+//   four MFMAs and a K fragment one of 32 rows.  P goes between them through
+//   LDS (8 KB per sub-tile).
+// The kernel is bound by what one wave per SIMD can issue.  A step's 68 MFMAs
+// take 2176 cycles and hide about six other instructions each; the step holds
+// some 480 and takes about 3400, 4600 cycles more go into a unit's first loads
+// and its output.  With 16 rows per wave in two passes of 64, QK^T, softmax and
+// PV one after the other and V^T read by every wave (the form before), 2176
+// cycles of MFMA took 12000.  Here step v holds QK^T of sub-tile v and PV of
+// sub-tile v - 1, which do not depend on each other, and the softmax of v runs
+// between the MFMAs of PV.  16 heads, us per call with the merge, before -> now:
+// 2921 prompt tokens of 5 requests (173 GFLOP) 419 -> 208; 1 x 2048 tokens 218 ->
+// 127; 8 x 64 tokens at 4096 keys 170 -> 100; 512 at 16K keys 264 (1089 TFLOP/s).
+// Keys go through LDS in sub-tiles of 32, a ring of three buffers filled by
+// direct loads a step ahead, one barrier per step.  Each wave computes the
+// cache slots of the keys it loads two steps ahead from the unit's block ids,
+// which are staged in LDS (2048 at a time) so that no load the compiler tracks
+// sits behind the direct loads in the loop (its wait would drain them).  A
+// unit's rows leave through LDS, a 1 KB store per row (stored from the
+// accumulators, 16 bytes of 32 rows at a time, the output took 10 us a unit).
+//   The order of a step is fixed in the source, one MFMA to a scheduling
+// region: left to itself the compiler waits for each LDS read in front of its
+// MFMA.  K fragments are read kMlaQkAhead MFMAs ahead, V^T fragments eight.
+// QK^T is issued as inline assembly because it accumulates in VGPRs while O
+// fills all 256 accumulation registers, a mix the compiler does not select
+// (with the builtin it moved 240 registers between the files every step).  The
+// hardware does not interlock a VALU read of an MFMA result: S is first read
+// after four PV MFMAs have been issued behind its last one (mla_s_ready).
+// LDS sub-tile: key r's 512 latent values, 64 16-byte chunks, chunk c at
+// c ^ f(r) with f(r) = 4 (r mod 4) + r / 4 mod 4: the 16 keys of a K fragment
+// read fall on 16 places, and so do the 4 keys x 4 chunks of a V^T read; then
+// the 64 rope values of every key, 128 bytes per key, chunk c at
+// c ^ (r / 2 mod 8).
 constexpr int kMlaSub = 32;                                       // keys per sub-tile
-constexpr int kMlaRing = 4;                                       // sub-tile buffers
-constexpr int kMlaAhead = kMlaRing - 1;                           // loads ahead
-constexpr int kMlaPfRow = 520;                                    // latent row stride (elements)
-constexpr int kMlaPfRope = kMlaSub * kMlaPfRow;                   // rope region offset
-constexpr int kMlaPfBuf = kMlaPfRope + kMlaSub * (kMlaK - kMlaV);   // elements per buffer
-constexpr int kMlaLoads = kMlaSub / kPfWaves + 1;                 // direct loads per wave
+constexpr int kMlaRing = 3;                                       // sub-tile buffers
+constexpr int kMlaPfRope = kMlaSub * kMlaV;                       // rope region offset (elements)
+constexpr int kMlaPfBuf = kMlaSub * kMlaK;                        // elements per buffer
 constexpr int kMlaBtl = 2048;                                     // staged block ids
-constexpr int kMlaKJ = kMlaK / 32;                                // 18 QK k-steps
-constexpr int kMlaDT = kMlaV / 16;                                // 32 output tiles
-constexpr int kMlaPassRows = kPfWaves * kRows;                    // 64 rows per pass
+constexpr int kMlaKJ = kMlaK / 16;                                // 36 QK k-steps
+constexpr int kMlaDT = 4;                                         // 32-dim output tiles per wave
+constexpr int kMlaRT = kPfRows / 32;                              // 32-row tiles per unit
+constexpr int kMlaQkAhead = 6;                                    // K fragments in flight
 constexpr float kMlaPfSpan = 64.f;   // log2 growth allowed over a row's reference max
 // s_waitcnt immediate: vmcnt(n) only (vmcnt bits 3:0 and 15:14)
 constexpr int wait_vmcnt(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 static_assert(wait_vmcnt(0) == kWaitVmcnt0, "s_waitcnt encoding");
-static_assert(kPfWaves == 4 && kPfKeys == 2 * kMlaSub && kPfRows % kMlaPassRows == 0 &&
-              kMlaV == 512 && kMlaK - kMlaV == 64 && kMlaSub == 8 * kPfWaves,
+static_assert(kPfWaves == 4 && kPfKeys == 2 * kMlaSub && kPfRows == 32 * kPfWaves &&
+              kMlaV == 128 * kPfWaves && kMlaK - kMlaV == 64 && kMlaSub == 8 * kPfWaves,
               "MLA prefill unit shape");
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+// S += K Q^T in VGPRs (see above); the first of a chain starts from zero.
+__device__ __forceinline__ void mla_s_first(float16_t& s, u32x4_t k, u32x4_t q) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "v"(q));
+}
+__device__ __forceinline__ void mla_s_next(float16_t& s, u32x4_t k, u32x4_t q) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "v"(q));
+}
+// S may be read from here on: NOPS covers an 8-pass MFMA's latency where no
+// other MFMA was issued after the chain.
+template <bool NOPS>
+__device__ __forceinline__ void mla_s_ready(float16_t& s) {
+  if (NOPS) asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s));
+  else asm volatile("" : "+v"(s));
+}
 
 __global__ __launch_bounds__(kPfWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mla_prefill_kernel(PrefillArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t ring[kMlaRing * kMlaPfBuf];
-  __shared__ int slots[kMlaRing][kMlaSub];
+  __shared__ __attribute__((aligned(16))) uint16_t pbuf[2 * kPfRows * kMlaSub];
   __shared__ int btl[kMlaBtl];
+  __shared__ float sl[kPfRows], sm[kPfRows], smax[kPfWaves][kPfRows];
   __shared__ int rerun_flag;
   const int wg = blockIdx.x;
   // this work-group's unit, as the GQA units take theirs (one kv head)
@@ -2887,234 +2922,351 @@ void mla_prefill_kernel(PrefillArgs a) {
   if (!whole && unit >= a.part_units) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = lane & 15, g = lane >> 4;
+  const int n = lane & 31, g = lane >> 5;
   const int32_t* btrow = a.bt + (int64_t)b * a.bt_stride;
   const int bs = a.bs;
+  const int u0 = 2 * t0, u1 = min(2 * t1, (kend + kMlaSub - 1) / kMlaSub);   // sub-tiles
+  const int nbk = (kend + bs - 1) / bs;               // blocks the unit may touch
 
-  // Wave 0: stage block ids [wb, wb + kMlaBtl) of the row (those below nbk)
-  int wb = -1;
-  auto stage_ids = [&](int first, int nbk) __attribute__((always_inline)) {
+  // Stage block ids [wb, wb + kMlaBtl) of the row (those below nbk),
+  // for the keys from sub-tile v on; vlim: the first sub-tile past them
+  int wb = 0, vlim = 0;
+  auto stage_ids = [&](int v) __attribute__((always_inline)) {
+    const int first = min(v * kMlaSub, kend - 1) / bs;
     wb = first;
-    for (int e = lane; e < kMlaBtl && first + e < nbk; e += 64)
+    vlim = (int64_t)(wb + kMlaBtl) * bs >= kend ? 0x7fffffff : (wb + kMlaBtl) * bs / kMlaSub;
+    for (int e = tid; e < kMlaBtl && first + e < nbk; e += kPfWaves * 64)
       btl[e] = min(max(btrow[first + e], 0), a.nb - 1);
   };
-  // Wave 0, lanes 0..31: cache slots of sub-tile v's keys (keys past the
-  // pass's last visible one re-read it)
-  auto make_slots = [&](int v, int kendp, int nbk) __attribute__((always_inline)) {
-    const int p = min(v * kMlaSub + lane, kendp - 1);
-    const int bi = p / bs;
-    if (__builtin_amdgcn_readfirstlane((v * kMlaSub) / bs) < wb ||
-        __builtin_amdgcn_readfirstlane(min(v * kMlaSub + kMlaSub, kendp) - 1) / bs >= wb + kMlaBtl)
-      stage_ids((v * kMlaSub) / bs, nbk);       // rare: a unit spanning more than kMlaBtl blocks
-    if (lane < kMlaSub) slots[v % kMlaRing][lane] = btl[bi - wb] * bs + (p - bi * bs);
+  // This lane's key of a sub-tile (wave w loads keys 8 w .. 8 w + 7, lane l
+  // stands for key 8 w + l / 8): its position, block and offset, advanced 32
+  // positions at a time; keys past the unit's last visible one re-read it.
+  const int rkey = 8 * wid + (lane >> 3);
+  const int adv_b = kMlaSub / bs, adv_o = kMlaSub - adv_b * bs;
+  const int last_b = max(kend - 1, 0) / bs, last_o = max(kend - 1, 0) - last_b * bs;
+  int kp = 0, kblk = 0, koff = 0;
+  auto first_key = [&](int v) __attribute__((always_inline)) {
+    kp = v * kMlaSub + rkey;
+    kblk = kp / bs;
+    koff = kp - kblk * bs;
   };
-  // Direct loads of sub-tile v into its ring buffer: wave w loads the latent
-  // of keys 8 w .. 8 w + 7 (one key per load, lane l its chunk l) and their
-  // rope (lane l chunk (l % 8) ^ (key % 8) of key 8 w + l / 8).
-  auto issue = [&](int v) __attribute__((always_inline)) {
-    uint16_t* dst = ring + (v % kMlaRing) * kMlaPfBuf;
-    const int* sl = slots[v % kMlaRing];
-#pragma unroll
-    for (int i = 0; i < kMlaSub / kPfWaves; ++i) {
-      const int r = wid * (kMlaSub / kPfWaves) + i;
-      const int slot = __builtin_amdgcn_readfirstlane(sl[r]);
-      aia::lds_load16(a.kc + (int64_t)slot * kMlaK + 8 * lane, dst + r * kMlaPfRow);
-    }
-    const int r = wid * (kMlaSub / kPfWaves) + (lane >> 3);
-    aia::lds_load16(a.kc + (int64_t)sl[r] * kMlaK + kMlaV + 8 * ((lane & 7) ^ (r & 7)),
-               dst + kMlaPfRope + wid * (kMlaSub / kPfWaves) * 64);
+  auto next_key = [&]() __attribute__((always_inline)) {
+    kp += kMlaSub;
+    kblk += adv_b;
+    koff += adv_o;
+    if (koff >= bs) { koff -= bs; ++kblk; }
   };
-
-  for (int pass = 0; pass < kPfRows / kMlaPassRows; ++pass) {
-    const int prow0 = row0 + pass * kMlaPassRows;
-    if (prow0 >= row_end) break;                      // uniform over the work-group
-    const int prow_end = min(row_end, prow0 + kMlaPassRows);
-    // keys this pass's last row sees, and its share of the unit's sub-tiles
-    const int kendp = max(0, min(lk, ctx0 + (prow_end - 1) / G + 1));
-    const int u0 = 2 * t0;
-    const int u1 = min(2 * t1, (kendp + kMlaSub - 1) / kMlaSub);
-    const int nbk = (kendp + bs - 1) / bs;            // blocks the pass may touch
-
-    const int row = prow0 + wid * kRows + n;
-    const bool rv = row < prow_end;
-    const int tokr = row / G, headr = row - tokr * G;
-    const int lim = rv ? min(ctx0 + tokr, lk - 1) : -1;
-    int wlim_lo = rv ? lim : 0x7fffffff, wlim_hi = lim;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      wlim_lo = min(wlim_lo, __shfl_xor(wlim_lo, d));
-      wlim_hi = max(wlim_hi, __shfl_xor(wlim_hi, d));
+  auto slot_of = [&]() __attribute__((always_inline)) {
+    const bool in = kp < kend;
+    return btl[(in ? kblk : last_b) - wb] * bs + (in ? koff : last_o);
+  };
+  // Direct loads of a sub-tile into a ring buffer, piece i of 9: the latent of
+  // key 8 w + i (lane l the chunk whose place is l), then the rope of all 8
+  // keys (lane l that of key 8 w + l / 8).
+  // lx = lane ^ (2 w mod 4): key 8 w + i's chunk for place l is lx ^ f(i).
+  auto issue = [&](int mine, int lx, int buf, int i) __attribute__((always_inline)) {
+    uint16_t* d = ring + buf * kMlaPfBuf;
+    if (i < 8) {
+      const int slot = __builtin_amdgcn_readlane(mine, 8 * i);
+      aia::lds_load16(a.kc + (int64_t)slot * kMlaK + 8 * (lx ^ (((i & 3) << 2) | (i >> 2))),
+                      d + (8 * wid + i) * kMlaV);
+    } else {
+      aia::lds_load16(a.kc + (int64_t)mine * kMlaK + kMlaV + 8 * ((lane & 7) ^ ((rkey >> 1) & 7)),
+                      d + kMlaPfRope + 8 * wid * 64);
     }
-    uint4 qf[kMlaKJ];
-    if (rv) {
-      const uint4* qp = reinterpret_cast<const uint4*>(
-          a.q + (int64_t)(q_begin + tokr) * a.q_ts + (int64_t)headr * a.q_hs);
+  };
+  const int lx0 = lane ^ (2 * (wid & 1));
+
+  // this wave's rows
+  const int row = row0 + 32 * wid + n;
+  const bool rv = row < row_end;
+  const int lim = rv ? min(ctx0 + row / G, lk - 1) : -1;
+  u32x4_t qf[kMlaKJ];
+  if (rv) {
+    const uint4* qp = reinterpret_cast<const uint4*>(
+        a.q + (int64_t)(q_begin + row / G) * a.q_ts + (int64_t)(row % G) * a.q_hs);
 #pragma unroll
-      for (int j = 0; j < kMlaKJ; ++j) qf[j] = qp[4 * j + g];
+    for (int j = 0; j < kMlaKJ; ++j) { qf[j] = as_u4(qp[2 * j + g]); }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kMlaKJ; ++j) qf[j] = u32x4_t{0, 0, 0, 0};
+  }
+
+  // LDS byte offsets within a sub-tile: K fragments of key n (chunk 2 j + g
+  // at kx ^ 32 (j mod 8) + 256 (j / 8)), its rope chunks (rx ^ 32 j), and V^T fragments:
+  // lane l of a 16-lane group addresses key 4 g + l / 4 (and + 8), dims 128 w +
+  // 32 dt + 16 h + 4 (l mod 4), at vx ^ 64 dt (and vx ^ 32 ^ 64 dt, + 8 keys)
+  const int fn = ((n & 3) << 2) | ((n >> 2) & 3);
+  const int kx0 = n * 1024 + 16 * (fn ^ g);
+  const int rx0 = kMlaPfRope * 2 + n * 128 + 16 * (((n >> 1) & 7) ^ g);
+  const int ll = lane & 15, vk = ll >> 2, vh = (lane >> 4) & 1;
+  const int vx0 = (4 * g + vk) * 1024 + 256 * wid +
+                 16 * ((2 * vh + ((ll >> 1) & 1)) ^ (4 * vk + g)) + 8 * (ll & 1);
+  const char* ringb = reinterpret_cast<const char*>(ring);
+  char* pb = reinterpret_cast<char*>(pbuf);
+
+  // Softmax without rescaling O: a row's reference m is its max over its
+  // first visible sub-tile, and later scores may exceed it by up to
+  // 2^kMlaPfSpan (P then stays a finite bf16, O and l finite fp32), so the
+  // loop holds no rescale branch.  A row whose scores climb further sets
+  // `ovf`, and the work-group then runs its sub-tiles again with every row's
+  // exact max as m (rmax, tracked on the way).
+  float16_t o[kMlaDT][kMlaRT];
+  float m = -INFINITY, lsum = 0.f, rmax = -INFINITY;
+  bool ovf = false;
+
+  // One step: QK^T of the sub-tile in buffer bk (if QK), PV of the one before
+  // it (v - 1, buffer bv; if PV), the softmax of v and its P.  With both, the
+  // loads of the next sub-tile go into buffer bn meanwhile (slots `mine`, then
+  // those of the sub-tile after it; past the unit's last key they re-read it).
+  // Without MASK every valid row sees all of sub-tile v's keys.
+  int mine = 0;          // this lane's slot in the sub-tile to load next
+  auto step = [&](auto qk_tag, auto pv_tag, auto mask_tag, int v, int bk, int bv, int bn)
+                  __attribute__((always_inline)) {
+    constexpr bool QK = decltype(qk_tag)::value, PV = decltype(pv_tag)::value;
+    constexpr bool MASK = decltype(mask_tag)::value;
+    // opaque copies, so that the swizzled offsets are computed where they are
+    // used (one xor each) instead of being kept, and spilled, across the loop
+    int kx = kx0, rx = rx0, vx = vx0, lx = lx0;
+    asm volatile("" : "+v"(kx), "+v"(rx), "+v"(vx), "+v"(lx));
+    const char* kt = ringb + bk * (kMlaPfBuf * 2);
+    const char* vt = ringb + bv * (kMlaPfBuf * 2);
+    const char* pp = pb + ((v - 1) & 1) * (kPfRows * kMlaSub * 2) + (g * kPfRows + n) * 16;
+    auto read_k = [&](int j) __attribute__((always_inline)) {
+      const char* p = j < kMlaV / 16 ? kt + ((kx ^ (32 * (j & 7))) + 256 * (j >> 3))
+                                     : kt + (rx ^ (32 * (j - kMlaV / 16)));
+      return *reinterpret_cast<const u32x4_t*>(p);
+    };
+    auto read_p = [&](int s, int rt) __attribute__((always_inline)) {
+      return *reinterpret_cast<const u32x4_t*>(pp + (2 * s * kPfRows + 32 * rt) * 16);
+    };
+    auto read_v = [&](int f) __attribute__((always_inline)) {       // fragment 4 s + dt
+      const int s = f >> 2, dt = f & 3;
+      const short4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4_t*)(vt + (vx ^ (64 * dt)) + s * 16384));
+      const short4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4_t*)(vt + (vx ^ 32 ^ (64 * dt)) + s * 16384 + 8192));
+      return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    u32x4_t pf[kMlaRT];
+    bf16x8_t vf[3];
+    auto pv_ahead = [&](int e) __attribute__((always_inline)) {     // PV's first operands, in 6 pieces
+      if (!PV) return;
+      if (e < 4) pf[e] = read_p(0, e);
+      else vf[e - 4] = read_v(e - 4);
+    };
+    float16_t acc;
+    if (QK) {
+      u32x4_t kf[kMlaQkAhead];
+#pragma unroll
+      for (int j = 0; j < kMlaQkAhead; ++j) kf[j] = read_k(j);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < kMlaKJ; ++j) {
+        if (j == 0) mla_s_first(acc, kf[0], qf[0]);
+        else mla_s_next(acc, kf[j % kMlaQkAhead], qf[j]);
+        if ((j & 7) == 1) asm volatile("" : "+v"(kx));
+        if (j + kMlaQkAhead < kMlaKJ) kf[j % kMlaQkAhead] = read_k(j + kMlaQkAhead);
+        else pv_ahead(j + kMlaQkAhead - kMlaKJ);
+        if (PV && j >= 2 && j < 29 && j % 3 == 2) issue(mine, lx, bn, (j - 2) / 3);
+        if (PV && j == 30) next_key();
+        if (PV && j == 31) mine = slot_of();
+        __builtin_amdgcn_sched_barrier(0);
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < kMlaKJ; ++j) qf[j] = make_uint4(0, 0, 0, 0);
+      for (int e = 0; e < 6; ++e) pv_ahead(e);
     }
-    // Softmax without rescaling O: a row's reference m is its max over its
-    // first visible sub-tile, and later scores may exceed it by up to
-    // 2^kMlaPfSpan (P then stays a finite bf16, O and l finite fp32), so the
-    // loop holds no rescale branch (one would keep O's 128 registers moving
-    // between register files every sub-tile).  A row whose scores climb
-    // further sets `ovf`, and the work-group then runs its sub-tiles again
-    // with every row's exact max as m (rmax, tracked on the way).
-    float4_t o[kMlaDT];
-    float m = -INFINITY, lsum = 0.f, rmax = -INFINITY;
-    bool ovf = false;
+    // softmax of v in 32 pieces, one to a PV MFMA
+    const int rel = lim - v * kMlaSub - 4 * g;
+    float p[16];
+    float tmax = -INFINITY, msub = 0.f, psum = 0.f;
+    uint32_t pk[8];
+    auto soft = [&](int i) __attribute__((always_inline)) {
+      if (!QK) return;
+      if (i == 3) mla_s_ready<!PV>(acc);
+      if (i >= 4 && i < 8) {
+#pragma unroll
+        for (int k = 4 * (i - 4); k < 4 * (i - 4) + 4; ++k) {
+          p[k] = !MASK || 8 * (k >> 2) + (k & 3) <= rel ? acc[k] : -INFINITY;
+          tmax = fmaxf(tmax, p[k]);
+        }
+      } else if (i == 8) {
+        tmax = aia::group2_max(tmax);
+        const float tm = tmax * a.scale_log2;
+        rmax = fmaxf(rmax, tm);
+        m = m == -INFINITY ? tm : m;                  // O and l are still zero
+        ovf = ovf || tm > m + kMlaPfSpan;
+        msub = m == -INFINITY ? 0.f : m;
+      } else if (i >= 9 && i < 25) {
+        const int k = i - 9;
+        p[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[k], a.scale_log2, -msub));
+        psum += p[k];
+        if (k & 1) pk[k >> 1] = aia::pack_bf16x2(p[k - 1], p[k]);
+      } else if (i == 25) {
+        lsum += psum;
+        // P in LDS: 16-byte pieces [step s][g][row], piece (s, g) holding keys
+        // 16 s + 4 g + {0..3, 8..11}: the order the V^T fragments take
+        char* d = pb + (v & 1) * (kPfRows * kMlaSub * 2) + (g * kPfRows + 32 * wid + n) * 16;
+        *reinterpret_cast<u32x4_t*>(d) = u32x4_t{pk[0], pk[1], pk[2], pk[3]};
+        *reinterpret_cast<u32x4_t*>(d + 2 * kPfRows * 16) = u32x4_t{pk[4], pk[5], pk[6], pk[7]};
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      if (PV) {
+        const int f = i >> 2, dt = f & 3, rt = i & 3;
+        o[dt][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[f % 3], __builtin_bit_cast(bf16x8_t, pf[rt]),
+                                                            o[dt][rt], 0, 0, 0);
+        if (i == 4) asm volatile("" : "+v"(vx));
+        if (rt == 3 && f + 3 < 8) vf[f % 3] = read_v(f + 3);
+        if (rt == 0 && f == 0) vf[2] = read_v(2);
+        if (f == 3) pf[rt] = read_p(1, rt);
+      }
+      soft(i);
+      if (PV) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto pin_o = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kMlaKJ; ++j) asm volatile("" : "+v"(qf[j]));
+#pragma unroll
+    for (int dt = 0; dt < kMlaDT; ++dt)
+#pragma unroll
+      for (int rt = 0; rt < kMlaRT; ++rt) asm volatile("" : "+a"(o[dt][rt]));
+  };
 
 #pragma clang loop unroll(disable)
-    for (int attempt = 0; attempt < 2; ++attempt) {
-      // O lives in the accumulation registers throughout (the empty asm
-      // pins it there; left to itself the compiler copied all 128 values
-      // between register files every sub-tile)
+  for (int attempt = 0; attempt < 2; ++attempt) {
 #pragma unroll
-      for (int dt = 0; dt < kMlaDT; ++dt) {
-        o[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
-        asm volatile("" : "+a"(o[dt]));
-      }
-      lsum = 0.f;
-      if (attempt > 0) { m = rmax; ovf = false; }   // every row's exact max
-      if (u1 > u0) {
-        // prologue: Q has arrived; slots of the first four sub-tiles, then
-        // the loads of the first three
+    for (int dt = 0; dt < kMlaDT; ++dt)
+#pragma unroll
+      for (int rt = 0; rt < kMlaRT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][rt][i] = 0.f;
+    pin_o();
+    lsum = 0.f;
+    if (attempt > 0) { m = rmax; ovf = false; }       // every row's exact max
+    if (u1 > u0) {
+      using yes = std::true_type;
+      using no = std::false_type;
+      // prologue: Q has arrived; block ids, then the first two sub-tiles
+      __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+      __syncthreads();                                // ring and block ids are free
+      stage_ids(u0);
+      __syncthreads();
+      first_key(u0);
+      mine = slot_of();
+#pragma unroll
+      for (int i = 0; i < 9; ++i) issue(mine, lx0, 0, i);
+      next_key();
+      mine = slot_of();
+#pragma unroll
+      for (int i = 0; i < 9; ++i) issue(mine, lx0, 1, i);
+      next_key();
+      mine = slot_of();
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt(9));      // sub-tile u0
+      __syncthreads();
+      step(yes{}, no{}, yes{}, u0, 0, 0, 0);
+      int bv = 0, bk = 1, bn = 2;                     // ring buffers of v - 1, v, v + 1
+      // sub-tiles that the unit's first token sees whole need no mask
+      const int v_um = (min(ctx0 + row0 / G, lk - 1) + 1) / kMlaSub;
+#pragma clang loop unroll(disable)
+      for (int v = u0 + 1; v < u1; ++v) {
+        // sub-tile v's loads have arrived and P of v - 1 is written; everyone
+        // has read sub-tile v - 2 and its P
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        __syncthreads();                              // the ring is free
-        if (wid == 0) {
-          wb = -1;
-          stage_ids((u0 * kMlaSub) / bs, nbk);
-          __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-          for (int v = u0; v < min(u1, u0 + kMlaRing); ++v) make_slots(v, kendp, nbk);
-        }
         __syncthreads();
-        for (int v = u0; v < min(u1, u0 + kMlaAhead); ++v) issue(v);
-#pragma clang loop unroll(disable)
-        for (int u = u0; u < u1; ++u) {
-          // sub-tile u's loads are the oldest of up to three in flight
-          const int younger = min(kMlaAhead - 1, u1 - 1 - u);
-          if (younger >= 2) __builtin_amdgcn_s_waitcnt(wait_vmcnt(2 * kMlaLoads));
-          else if (younger == 1) __builtin_amdgcn_s_waitcnt(wait_vmcnt(kMlaLoads));
-          else __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+        if (v + 2 >= vlim) {                          // rare: past the staged block ids
           __syncthreads();
-          const uint16_t* kt = ring + (u % kMlaRing) * kMlaPfBuf;
-          const int kb = u * kMlaSub;
-          if (kb <= wlim_hi) {                        // some row of this wave sees the keys
-            float4_t acc[2];
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-              const int r = 16 * s2 + n;
-              const uint16_t* kl = kt + r * kMlaPfRow + 8 * g;
-              float4_t part[4];
-#pragma unroll
-              for (int c4 = 0; c4 < 4; ++c4) part[c4] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-              for (int j = 0; j < kMlaKJ - 2; ++j)
-                part[j & 3] = qk_step(*reinterpret_cast<const uint4*>(kl + 32 * j), qf[j], part[j & 3]);
-#pragma unroll
-              for (int j = kMlaKJ - 2; j < kMlaKJ; ++j) {
-                const int c = (4 * (j - (kMlaKJ - 2)) + g) ^ (r & 7);
-                part[j & 3] = qk_step(*reinterpret_cast<const uint4*>(kt + kMlaPfRope + r * 64 + 8 * c),
-                                      qf[j], part[j & 3]);
-              }
-              acc[s2] = (part[0] + part[1]) + (part[2] + part[3]);
-            }
-            if (u + kMlaAhead < u1) issue(u + kMlaAhead);
-            const bool mask = kb + kMlaSub - 1 > wlim_lo;
-            float sv[2][4];
-            float tmax = -INFINITY;
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-              for (int v = 0; v < 4; ++v) {
-                sv[s2][v] = (mask && kb + 16 * s2 + 4 * g + v > lim) ? -INFINITY : acc[s2][v];
-                tmax = fmaxf(tmax, sv[s2][v]);
-              }
-            tmax = aia::group4_max(tmax);
-            const float tm = tmax * a.scale_log2;
-            rmax = fmaxf(rmax, tm);
-            if (m == -INFINITY) m = tm;               // O and l are still zero
-            ovf = ovf || tm > m + kMlaPfSpan;
-            const float msub = m == -INFINITY ? 0.f : m;
-            float p[2][4];
-            float psum = 0.f;
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-              for (int v = 0; v < 4; ++v) {
-                p[s2][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[s2][v], a.scale_log2, -msub));
-                psum += p[s2][v];
-              }
-            lsum += psum;
-            uint4 pb;
-            pb.x = aia::pack_bf16x2(p[0][0], p[0][1]);
-            pb.y = aia::pack_bf16x2(p[0][2], p[0][3]);
-            pb.z = aia::pack_bf16x2(p[1][0], p[1][1]);
-            pb.w = aia::pack_bf16x2(p[1][2], p[1][3]);
-            // PV: lane (n, g) addresses key 4 g + n / 4 (and + 16), dims
-            // 16 dt + 4 (n % 4)
-            const uint16_t* v0p = kt + (4 * g + (n >> 2)) * kMlaPfRow + 4 * (n & 3);
-            const uint16_t* v1p = v0p + 16 * kMlaPfRow;
-#pragma unroll
-            for (int dt = 0; dt < kMlaDT; ++dt) {
-              const short4_t x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(v0p + 16 * dt));
-              const short4_t x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(v1p + 16 * dt));
-              const bf16x8_t va = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
-              o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, as_b8(pb), o[dt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int dt = 0; dt < kMlaDT; ++dt) asm volatile("" : "+a"(o[dt]));
-          } else if (u + kMlaAhead < u1) {
-            issue(u + kMlaAhead);
-          }
-          // slots of sub-tile u + 4 into the ring slot sub-tile u's loads used
-          if (wid == 0 && u + kMlaRing < u1) make_slots(u + kMlaRing, kendp, nbk);
+          stage_ids(v + 2);
+          __syncthreads();
         }
+        if (v < v_um) step(yes{}, yes{}, no{}, v, bk, bv, bn);
+        else step(yes{}, yes{}, yes{}, v, bk, bv, bn);
+        pin_o();
+        const int t = bv;
+        bv = bk; bk = bn; bn = t;
       }
-      // a row past its reference span: the work-group runs its sub-tiles again
-      if (tid == 0) rerun_flag = 0;
+      __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);       // no load outlives the ring's use
       __syncthreads();
-      if (__any(ovf) && lane == 0) rerun_flag = 1;
-      __syncthreads();
-      const int rerun = rerun_flag;
-      __syncthreads();
-      if (!rerun) break;
+      step(no{}, yes{}, no{}, u1, 0, bv, 0);
+      pin_o();
     }
+    // a row past its reference span: the work-group runs its sub-tiles again
+    if (tid == 0) rerun_flag = 0;
+    __syncthreads();
+    if (__any(ovf) && lane == 0) rerun_flag = 1;
+    __syncthreads();
+    const int rerun = rerun_flag;
+    __syncthreads();
+    if (!rerun) break;
+  }
 
-    lsum = aia::group4_sum(lsum);
-    float cmax = 0.f;
-    if (!whole) {
+  // every row's l (m), and the scale of its partial, to all waves
+  lsum = aia::group2_sum(lsum);
+  if (g == 0) { sl[32 * wid + n] = lsum; sm[32 * wid + n] = m; }
+  if (!whole) {
+#pragma unroll
+    for (int rt = 0; rt < kMlaRT; ++rt) {
+      float cmax = 0.f;
 #pragma unroll
       for (int dt = 0; dt < kMlaDT; ++dt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) cmax = fmaxf(cmax, fabsf(o[dt][v]));
-      cmax = aia::group4_max(cmax);
+        for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, fabsf(o[dt][rt][i]));
+      cmax = aia::group2_max(cmax);
+      if (g == 0) smax[wid][32 * rt + n] = cmax;
     }
-    if (!rv) continue;
-    if (!whole) {      // partial: y = O / c in fp16, (m + log2 c, l / c)
-      const float c = cmax > 0.f ? cmax : 1.f, ic = 1.f / c;
-      const int64_t prow = (int64_t)unit * kPfRows + (row - row0);
-      uint16_t* pp = a.part_o + prow * kMlaV;
+  }
+  __syncthreads();
+  // Rows go out through LDS, 64 at a time in the ring (rows of 1040 bytes), so
+  // that a store covers a row's 1 KB instead of 16 bytes of 32 rows: bf16
+  // outputs, or a partial y = O / c in fp16 with (m + log2 c, l / c).
+  constexpr int kOutRow = 1040;
+  char* ob = reinterpret_cast<char*>(ring);
 #pragma unroll
-      for (int dt = 0; dt < kMlaDT; ++dt) {
-        uint2 hv;
-        hv.x = pack_f16x2(o[dt][0] * ic, o[dt][1] * ic);
-        hv.y = pack_f16x2(o[dt][2] * ic, o[dt][3] * ic);
-        *reinterpret_cast<uint2*>(pp + 16 * dt + 4 * g) = hv;
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();
+#pragma unroll
+    for (int rt = 2 * half; rt < 2 * half + 2; ++rt) {
+      const int r = 32 * rt + n;
+      char* d = ob + (r - 64 * half) * kOutRow + 2 * (128 * wid + 4 * g);
+      if (!whole) {
+        const float cm = fmaxf(fmaxf(smax[0][r], smax[1][r]), fmaxf(smax[2][r], smax[3][r]));
+        const float c = cm > 0.f ? cm : 1.f, ic = 1.f / c;
+#pragma unroll
+        for (int dt = 0; dt < kMlaDT; ++dt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint2 hv;
+            hv.x = pack_f16x2(o[dt][rt][4 * q] * ic, o[dt][rt][4 * q + 1] * ic);
+            hv.y = pack_f16x2(o[dt][rt][4 * q + 2] * ic, o[dt][rt][4 * q + 3] * ic);
+            *reinterpret_cast<uint2*>(d + 2 * (32 * dt + 8 * q)) = hv;
+          }
+        if (g == 0 && wid == 0 && row0 + r < row_end)
+          a.part_ml[(int64_t)unit * kPfRows + r] = make_float2(sm[r] + __log2f(c), sl[r] * ic);
+      } else {
+        const float l = sl[r], inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int dt = 0; dt < kMlaDT; ++dt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint2 wv;
+            wv.x = aia::pack_bf16x2(o[dt][rt][4 * q] * inv, o[dt][rt][4 * q + 1] * inv);
+            wv.y = aia::pack_bf16x2(o[dt][rt][4 * q + 2] * inv, o[dt][rt][4 * q + 3] * inv);
+            *reinterpret_cast<uint2*>(d + 2 * (32 * dt + 8 * q)) = wv;
+          }
       }
-      if (g == 0) a.part_ml[prow] = make_float2(m + __log2f(c), lsum * ic);
-      continue;
     }
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    uint16_t* op = a.out + (int64_t)(q_begin + tokr) * a.o_ts + (int64_t)headr * a.o_hs;
-#pragma unroll
-    for (int dt = 0; dt < kMlaDT; ++dt) {
-      uint2 wv;
-      wv.x = aia::pack_bf16x2(o[dt][0] * inv, o[dt][1] * inv);
-      wv.y = aia::pack_bf16x2(o[dt][2] * inv, o[dt][3] * inv);
-      *reinterpret_cast<uint2*>(op + 16 * dt + 4 * g) = wv;
+    __syncthreads();
+#pragma unroll 4
+    for (int i = 0; i < 16; ++i) {
+      const int r = 64 * half + 16 * wid + i, orow = row0 + r;
+      if (orow >= row_end) break;                     // uniform over the wave
+      const uint4 x = *reinterpret_cast<const uint4*>(ob + (16 * wid + i) * kOutRow + 16 * lane);
+      uint16_t* dst = whole ? a.out + (int64_t)(q_begin + orow / G) * a.o_ts + (int64_t)(orow % G) * a.o_hs
+                            : a.part_o + ((int64_t)unit * kPfRows + r) * kMlaV;
+      reinterpret_cast<uint4*>(dst)[lane] = x;
     }
   }
 }

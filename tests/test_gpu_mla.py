@@ -222,18 +222,23 @@ def test_mla_prefill_row_blocks(lqs, lks, heads, bs, waves):
 
 
 # MLA prefill units (requests of 8+ tokens, 4+ tokens per request on
-# average): 128-row items in two 64-row passes, 32-key sub-tiles in a ring
-# of four LDS buffers.  Cases: units cut into key chunks (partials and the
-# chunk merge), one request against 16K keys, a block size of 4 with more
-# than 2048 blocks under one unit (the staged block ids are replaced
-# mid-unit), units beside split-K rows, and scores spread so wide that a
-# row exceeds its reference max by 2^64 (the unit runs its tiles again).
+# average): 128-row items, 32-key sub-tiles in a ring of three LDS buffers.
+# Cases: units cut into key chunks (partials and the chunk merge), one
+# request against 16K keys, more than 2048 blocks under one unit (the staged
+# block ids are replaced mid-unit), units beside split-K rows, 1 to 130 keys
+# (one sub-tile, and a last one of one key), 1 to 64 heads (units of 128 to 2
+# tokens), and scores spread so wide that a row exceeds its reference max by
+# 2^64 (the unit runs its tiles again).
 @pytest.mark.parametrize("lqs,lks,bs,heads", [
     ([64] * 8, [4096] * 8, 128, 16),
     ([512], [16384], 128, 16),
     ([64], [12000], 4, 16),
     ([40, 1, 1, 9, 24], [2000, 300, 5000, 9, 24 + 700], 16, 16),
     ([16] * 6, [((i * 777) % 3000) + 16 for i in range(6)], 64, 32),
+    ([900], [2600], 1, 64),
+    ([8, 31, 32, 33, 65, 130], [8, 31, 32, 33, 65, 130], 16, 16),
+    ([200, 129], [233, 129], 32, 1),
+    ([100, 43], [101, 700], 7, 3),
 ])
 def test_mla_prefill_units(lqs, lks, bs, heads):
     print(f"mla prefill units lqs={lqs[:5]} lks={lks[:5]} bs={bs} heads={heads}", flush=True)

@@ -175,6 +175,14 @@ Geometry geometry(int32_t hq, int32_t hkv, int32_t batch, int32_t tokens, int32_
   return g;
 }
 
+#ifndef AIA_MIXED
+#define AIA_MIXED 1
+#endif
+// Prefill units and split-K ranges of a step run in one grid (gqa_mixed_kernel).
+__host__ __device__ inline bool mixed_grid(const Geometry& g, int32_t dv) {
+  return AIA_MIXED && g.pf && g.nw == kPfWaves && g.rb == 1 && dv == kHeadDim;
+}
+
 // Workspace layout (all offsets 256-byte aligned).
 struct Layout {
   int64_t hdr, seg, wave, part_ml, part_o, req, mrg, pf, pfm, pfw, pf_o, pf_ml, total;
@@ -237,15 +245,16 @@ Layout layout(int32_t batch, int32_t tokens, const Geometry& g, int32_t dv, int3
   const int64_t pf_rows = g.pf ? (int64_t)tokens * g.group : 0;
   const int64_t pf_reqs = pf_rows / kPfRows < batch ? pf_rows / kPfRows : batch;
   L.pf_cap = (pf_rows + kPfRows - 1) / kPfRows + pf_reqs;
-  // Chunked items exist only when items x kv heads < kPfTargetWgs; then the
-  // units number at most items + total tiles / chunk < 2 kPfTargetWgs / Hkv.
+  // Items are cut only while their units x kv heads stay within kPfTargetWgs
+  // or two work-groups per CU (512), and a cut item has two units or more.
+  static_assert(2 * kPfTargetWgs >= 512, "partial row blocks for two work-groups per CU");
   const int64_t split_units = g.pf ? 2 * ((kPfTargetWgs + g.hkv - 1) / g.hkv) + 1 : 0;
   L.pf_unit_cap = L.pf_cap > split_units ? L.pf_cap : split_units;
   L.pf_mrg_cap = g.pf ? (kPfTargetWgs + g.hkv - 1) / g.hkv : 0;
   L.pf_slots = split_units * g.hkv;             // partial row blocks
   L.pf = off;       off = align256(off + L.pf_unit_cap * 32);              // two int4 per unit
   L.pfm = off;      off = align256(off + L.pf_mrg_cap * 16);
-  L.pfw = off;      off = align256(off + (g.pf ? kPfTargetWgs * 48 : 0));   // dealt work-groups
+  L.pfw = off;      off = align256(off + L.pf_unit_cap * g.hkv * 48);   // dealt work-groups
   L.pf_ml = off;    off = align256(off + L.pf_slots * kPfRows * 8);
   L.pf_o = off;     off = align256(off + L.pf_slots * kPfRows * (int64_t)dv * 2);
   L.total = off;
@@ -457,28 +466,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       const int kend = max(0, min(lk, lk - lq + last / g.group + 1));
       return (kend + kPfKeys - 1) / kPfKeys;
     };
-    int chunk = 0x7fffffff;
-    if ((int64_t)pcarry * g.hkv < pf_target) {
-      int mine = 0;
-      for (int f = tid; f < pcarry; f += kPlanThreads) {
-        int b, r0;
-        mine += item_at(f, b, r0);
-      }
-      int wtot;
-      block_exclusive_scan(mine, wave_sums, &wtot);
-      // sum_i ceil(nt_i / c) <= W / c + P, so c = W Hkv / (target - P Hkv)
-      // keeps units x kv heads within the target: one round of work-groups
-      const int64_t room = pf_target - (int64_t)pcarry * g.hkv;
-      chunk = max(kPfMinChunk, (int)(((int64_t)wtot * g.hkv + room - 1) / room));
-      // That bound is loose.  In a step with no split-K segments the least
-      // chunk whose units still fit evens the work-groups out (the slowest
-      // one sets the kernel time), found by a binary search, one block
-      // reduction per probe.  Beside split-K ranges the loose bound stays:
-      // its fewer work-groups leave slots for the HBM-bound ranges.
-      const int ucap = pf_target / g.hkv;
-      int lo = carry > 0 ? chunk : max(kPfMinChunk, (wtot + ucap - 1) / ucap);
-      while (lo < chunk) {
-        const int mid = (lo + chunk) >> 1;
+    int chunk = 0x7fffffff, wtot = 0;
+    // the least chunk above `lo` and up to `hi` whose units number at most ucap
+    auto least_chunk = [&](int lo, int hi, int ucap) {
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
         int nu = 0;
         for (int f = tid; f < pcarry; f += kPlanThreads) {
           int b, r0;
@@ -487,8 +479,55 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         }
         int utot;
         block_exclusive_scan(nu, wave_sums, &utot);
-        if (utot <= ucap) chunk = mid; else lo = mid + 1;
+        if (utot <= ucap) hi = mid; else lo = mid + 1;
       }
+      return hi;
+    };
+    // The prefill work-groups have the chip to themselves when nothing is
+    // left to the split-K kernel or it is launched on its own.
+    const int pair_slots = min(2 * g.ncu, 512);
+    const bool alone = carry == 0 || (dv != 512 && !mixed_grid(g, dv));
+    const bool even = dv != 512 && alone && (int64_t)pcarry * g.hkv < pair_slots;
+    int mine = 0, most = 0;
+    for (int f = tid; f < pcarry; f += kPlanThreads) {
+      int b, r0;
+      const int nt = item_at(f, b, r0);
+      mine += nt;
+      most = max(most, nt);
+    }
+    block_exclusive_scan(mine, wave_sums, &wtot);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
+    if (tid == 0) pf_hist[0] = 0;
+    __syncthreads();
+    if ((tid & 63) == 0) atomicMax(&pf_hist[0], most);
+    __syncthreads();
+    const int longest = pf_hist[0];                  // tiles of the longest item
+    __syncthreads();
+    if ((int64_t)pcarry * g.hkv < pf_target) {
+      // sum_i ceil(nt_i / c) <= W / c + P, so c = W Hkv / (target - P Hkv)
+      // keeps units x kv heads within the target: one round of work-groups
+      const int64_t room = pf_target - (int64_t)pcarry * g.hkv;
+      chunk = max(kPfMinChunk, (int)(((int64_t)wtot * g.hkv + room - 1) / room));
+      // That bound is loose.  Alone on the chip, the least chunk whose units
+      // still fit evens the work-groups out (the slowest one sets the kernel
+      // time), found by a binary search, one block reduction per probe.
+      // Beside split-K ranges the loose bound stays: its fewer work-groups
+      // leave slots for the HBM-bound ranges.
+      const int ucap = pf_target / g.hkv;
+      if (alone) chunk = least_chunk(max(kPfMinChunk, (wtot + ucap - 1) / ucap), chunk, ucap);
+    }
+    // Ragged prompts: items that nearly fill the target are left (almost)
+    // uncut by it, and the longest sets the kernel time.  They are cut for
+    // two work-groups per CU where that shortens the longest by an eighth (7
+    // prompts of 40 to 1657 tokens, 14 / 2 heads of 64: 37.0 us per call to
+    // 30.5; 4 chunks of 512 tokens at 4096 keys, whose items are all long,
+    // 126 uncut and 130 cut; 768 or more work-groups 3 - 10 us slower on
+    // either).
+    if (even) {
+      const int ucap = pair_slots / g.hkv, top = min(longest, chunk);
+      const int c2 = least_chunk(min(top, max(kPfMinChunk, (wtot + ucap - 1) / ucap)), top, ucap);
+      if (8 * c2 <= 7 * top) chunk = c2;
     }
     int ucarry = 0, mcarry2 = 0;
     for (int base = 0; base < pcarry; base += kPlanThreads) {
@@ -531,27 +570,35 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
 
     // 1c) Work-group b's record at pf_wg[b]: its unit record (two int4),
     // then {unit, kv head}, so a work-group loads it beside the header
-    // instead of after it; hdr[9] = the number written (0: too many
-    // work-groups, they read the unit list).  When a step has only prefill
-    // work-groups and they fit one round, two per CU (the hardware puts
-    // work-groups b and b + ncu on one CU then), they are dealt by size so
-    // every CU's pair sums evenly: the largest units alone on the CUs
-    // without a partner, then the i-th largest of the rest beside the i-th
-    // smallest.  Otherwise b takes (kv head, unit) pair xcd_range(b, pairs):
-    // each XCD gets a contiguous run of pairs, kv-head major, so the items
-    // that re-read one request's keys for one kv head share an XCD's L2.
+    // instead of after it; hdr[9] = the number written.  Work-groups go to
+    // the XCDs round-robin by id, so b takes XCD b % 8.
+    // - Prefill work-groups alone on the chip that fit one round, two per CU
+    //   (the hardware puts work-groups b and b + ncu on one CU then), are
+    //   dealt by size so every CU's pair sums evenly: the largest units alone
+    //   on the CUs without a partner, then the i-th largest of the rest
+    //   beside the i-th smallest.
+    // - In more than one round the next work-group goes to whichever CU frees
+    //   first, so they are dealt largest first.  Each kv head's work-groups
+    //   stay on its XCDs (8 / Hkv of them, or Hkv / 8 heads on one), whose L2
+    //   the items that re-read its keys share, every XCD of a head taking
+    //   every (8 / Hkv)-th size.  In list order the XCDs' runs differ by the
+    //   prompts' lengths and long items start last: us per call, list order
+    //   to dealt, 8 prompts of up to 3559 tokens, 14 / 2 heads of 64: 131 to
+    //   90; 6 of up to 1896, 8 / 1: 121 to 84; 5 of up to 1813, 28 / 4: 146
+    //   to 116; one of 16384: 2170 to 1706; 3 of up to 2141, 64 / 8: 182 to
+    //   178.  One size order over all heads: 84, 124, -, 185.
+    // - Else (one work-group per CU or less, or beside split-K ranges) each
+    //   XCD gets a contiguous run of (kv head, unit) pairs, kv-head major.
+    // Absorbed-MLA units run one per CU and are always dealt largest first.
     const int jobs = units * g.hkv;
-    // Absorbed-MLA units run one per CU: in more than one round the next
-    // work-group goes to whichever CU frees first, so they are dealt largest
-    // first (the longest-processing-time order).
-    const bool lpt = dv == 512 && AIA_MLA_LPT;
-    const bool pair_deal = !lpt && carry == 0 && jobs > g.ncu && jobs <= 2 * g.ncu;
-    if (jobs <= pf_target && !pair_deal && !lpt) {
+    const bool lpt = (dv == 512 && AIA_MLA_LPT) || jobs > 2 * g.ncu;
+    const bool pair_deal = !lpt && alone && jobs > g.ncu && jobs <= 2 * g.ncu;
+    if (!pair_deal && !lpt) {
       __syncthreads();   // publishes pf_units to the whole group
       const int q = jobs / kXcdsPlan, r = jobs - q * kXcdsPlan;
       for (int id = tid; id < jobs; id += kPlanThreads) {
         const int x = id % kXcdsPlan, i = id / kXcdsPlan;
-        const int pair = x * q + min(x, r) + i;          // xcd_range(id, jobs)
+        const int pair = x * q + min(x, r) + i;          // the run of XCD id % 8
         const int kvh = pair / units, u = pair - kvh * units;
         pf_wg[3 * id] = pf_units[2 * u];
         pf_wg[3 * id + 1] = pf_units[2 * u + 1];
@@ -559,12 +606,15 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       }
       dealt = jobs;
     }
-    if ((pair_deal || lpt) && jobs <= pf_target) {
+    if (pair_deal || lpt) {
       if (tid < 64) pf_hist[tid] = 0;
       __syncthreads();   // also publishes pf_units to the whole group
-      for (int p = tid; p < jobs; p += kPlanThreads) {
+      // 64 buckets of sizes up to the longest item's, bucket 0 the largest
+      auto bucket = [&](int nt) { return 63 - (int)min(64u * (unsigned)nt / (unsigned)(longest + 1), 63u); };
+      const int heads = lpt ? 1 : g.hkv, listed = units * heads;   // pairs sorted
+      for (int p = tid; p < listed; p += kPlanThreads) {
         const int4 e = pf_units[2 * (p % units)];
-        atomicAdd(&pf_hist[63 - min(e.w - e.z, 63)], 1);   // bucket 0: the largest
+        atomicAdd(&pf_hist[bucket(e.w - e.z)], 1);
       }
       __syncthreads();
       if (tid == 0) {
@@ -573,15 +623,30 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       }
       __syncthreads();
       const int n2 = jobs - g.ncu, lone = g.ncu - n2;
-      for (int p = tid; p < jobs; p += kPlanThreads) {
-        const int u = p % units, kvh = p / units;
-        const int4 e = pf_units[2 * u];
-        const int r = atomicAdd(&pf_hist[63 - min(e.w - e.z, 63)], 1);
-        const int i = r - lone;
-        const int id = lpt ? r : r < lone ? n2 + r : i < n2 ? i : g.ncu + (jobs - 1 - r);
-        pf_wg[3 * id] = e;
-        pf_wg[3 * id + 1] = pf_units[2 * u + 1];
-        pf_wg[3 * id + 2] = make_int4(u, kvh, 0, 0);
+      const int per = kXcdsPlan / g.hkv, hpx = g.hkv / kXcdsPlan;
+      for (int p = tid; p < listed; p += kPlanThreads) {
+        const int u = p % units;
+        const int4 e = pf_units[2 * u], e2 = pf_units[2 * u + 1];
+        const int r = atomicAdd(&pf_hist[bucket(e.w - e.z)], 1);
+        auto put = [&](int id, int kvh) {
+          pf_wg[3 * id] = e;
+          pf_wg[3 * id + 1] = e2;
+          pf_wg[3 * id + 2] = make_int4(u, kvh, 0, 0);
+        };
+        if (!lpt) {
+          const int i = r - lone;
+          put(r < lone ? n2 + r : i < n2 ? i : g.ncu + (jobs - 1 - r), p / units);
+          continue;
+        }
+        for (int kvh = 0; kvh < g.hkv; ++kvh) {
+          int id = r * g.hkv + kvh;
+          if (hpx * kXcdsPlan == g.hkv) {
+            id = kXcdsPlan * (r * hpx + kvh % hpx) + kvh / hpx;
+          } else if (per * g.hkv == kXcdsPlan && r < units - units % per) {
+            id = kXcdsPlan * (r / per) + kvh * per + r % per;
+          }
+          put(id, kvh);
+        }
       }
       dealt = jobs;
     }
@@ -1504,20 +1569,6 @@ __device__ __forceinline__ void gqa_segment(const AttnArgs& a, const int* rec, i
   }
 }
 
-// XCD-aware order of the prefill work items.  The hardware deals
-// work-groups to the 8 XCDs round-robin by id; mapping work-group b to item
-// x q + min(x, r) + b / 8 (x = b % 8, n = 8 q + r) gives each XCD a
-// contiguous run of items, so the requests it serves -- and the keys their
-// query blocks re-read -- stay in its own L2.  (The split-K ranges get the
-// same order from the planner, which writes them into their slots.)
-constexpr int kXcds = 8;
-static_assert(kXcds == kXcdsPlan, "one XCD count for the planner and the kernels");
-__device__ __forceinline__ int xcd_range(int b, int n) {
-  const int q = n / kXcds, r = n - q * kXcds;
-  const int x = b % kXcds, i = b / kXcds;
-  return x * q + min(x, r) + i;
-}
-
 // One work-group per key range, one wave per kv head of the segment's group.
 // D: head dim, 128 or 64.
 template <int NW, int RB, int D, bool NZ>
@@ -1589,10 +1640,9 @@ struct PrefillArgs {
   float scale_log2;
   uint16_t* out;
   int64_t o_ts, o_hs;
-  const int4* units;         // per unit: {request, first row, first tile, end tile},
-                             // {first query token, query tokens, keys, first tile's block id}
-  const int4* dealt;         // work-group b: its unit record (two int4), then {unit, kv head}
-                             // (written when the work-groups fit kPfTargetWgs, hdr[9])
+  const int4* dealt;         // work-group b: {request, first row, first tile, end tile},
+                             // {first query token, query tokens, keys, first tile's block id},
+                             // {unit, kv head}
   const int32_t* hdr;
   uint16_t* part_o;          // partial row blocks of chunked items (fp16, scaled per row)
   float2* part_ml;
@@ -1646,39 +1696,15 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
   constexpr int KJ = D / 32;        // 32-dim MFMA k-steps
   constexpr int DT = D / 16;        // 16-dim output tiles
   constexpr int RC = D / 8;         // 16-byte chunks per K / V row
-  // The planner writes work-group b's record at dealt[b] when the
-  // work-groups fit the fill target (hdr[9] = their number; dealt by size, or
-  // in xcd_range order); it is loaded beside the header rather than after
-  // it.  Past the target, work-group b takes (kv head, item) pair
-  // xcd_range(b, pairs), kv-head major: each XCD gets a contiguous run of
-  // pairs, so the items that re-read one request's keys for one kv head
-  // share an XCD's L2.
-  int4 w0 = make_int4(0, 0, 0, 0), w1 = w0, w2 = w0;
-  if (wg < kPfTargetWgs) {
-    w0 = a.dealt[3 * wg];
-    w1 = a.dealt[3 * wg + 1];
-    w2 = a.dealt[3 * wg + 2];
-  }
+  // The planner writes work-group b's record at dealt[b] (the grid is as long
+  // as the list can be); it is loaded beside the header rather than after it.
+  const int4 it = a.dealt[3 * wg], iq = a.dealt[3 * wg + 1], uk = a.dealt[3 * wg + 2];
   const int count = a.hdr[6];
-  const int pairs = count * a.hkv;
-  if (wg >= pairs) return;
-  int kvh, unit;
-  int4 it, iq;
-  if (a.hdr[9] == pairs) {     // this work-group's record (see the planner)
-    it = w0;
-    iq = w1;
-    unit = w2.x;
-    kvh = w2.y;
-    if (unit < 0 || unit >= count) return;
-  } else {
-    const int pair = xcd_range(wg, pairs);
-    kvh = pair / count;
-    unit = pair - kvh * count;
-    it = a.units[2 * unit];
-    iq = a.units[2 * unit + 1];
-  }
+  if (wg >= count * a.hkv) return;
+  const int unit = uk.x, kvh = uk.y;
+  if (unit < 0 || unit >= count) return;
   const int b = it.x, row0 = it.y, t0 = it.z, t1 = it.w;
-  if (b < 0 || b >= a.batch || kvh >= a.hkv) return;
+  if (b < 0 || b >= a.batch || kvh < 0 || kvh >= a.hkv) return;
   const int q_begin = iq.x, lq = iq.y, lk = iq.z, bid0 = iq.w;
   const int G = a.group;
   const int nrows = lq * G;
@@ -2090,9 +2116,6 @@ void gqa_prefill_kernel(PrefillArgs a) {
 // 512, so the second kernel mostly waits for the first to drain.  In one grid every
 // work-group gets the prefill budget and does one job or the other, so the
 // compute-bound prefill runs while the HBM-bound decode streams beside it.
-#ifndef AIA_MIXED
-#define AIA_MIXED 1
-#endif
 // The decode role stages its V^T tiles in the first K buffer.
 constexpr int kMixedK0 = kPfWaves * kTile * kVStride > kPfKeys * kKStride
                              ? kPfWaves * kTile * kVStride : kPfKeys * kKStride;
@@ -2887,26 +2910,11 @@ void mla_prefill_kernel(PrefillArgs a) {
   __shared__ int rerun_flag;
   const int wg = blockIdx.x;
   // this work-group's unit, as the GQA units take theirs (one kv head)
-  int4 w0 = make_int4(0, 0, 0, 0), w1 = w0, w2 = w0;
-  if (wg < kPfTargetWgs) {
-    w0 = a.dealt[3 * wg];
-    w1 = a.dealt[3 * wg + 1];
-    w2 = a.dealt[3 * wg + 2];
-  }
+  const int4 it = a.dealt[3 * wg], iq = a.dealt[3 * wg + 1];
+  const int unit = a.dealt[3 * wg + 2].x;
   const int count = a.hdr[6];
   if (wg >= count) return;
-  int unit;
-  int4 it, iq;
-  if (a.hdr[9] == count) {
-    it = w0;
-    iq = w1;
-    unit = w2.x;
-    if (unit < 0 || unit >= count) return;
-  } else {
-    unit = xcd_range(wg, count);
-    it = a.units[2 * unit];
-    iq = a.units[2 * unit + 1];
-  }
+  if (unit < 0 || unit >= count) return;
   const int b = it.x, row0 = it.y, t0 = it.z, t1 = it.w;
   if (b < 0 || b >= a.batch) return;
   const int q_begin = iq.x, lq = iq.y, lk = iq.z;
@@ -3359,7 +3367,7 @@ template <bool NZ>
 int launch_gqa(const AttnArgs& a, const PrefillArgs& pa, const Layout& L, const Geometry& g,
                int32_t head_dim, int32_t waves, bool one_block, hipStream_t s) {
   using aia::check_hip;
-  if (AIA_MIXED && L.pf_cap > 0 && g.nw == kPfWaves && g.rb == 1 && head_dim == kHeadDim) {
+  if (mixed_grid(g, head_dim)) {
     const int npf = (int)(L.pf_unit_cap * g.hkv);
     const dim3 grid((unsigned)(npf + waves));
     if (one_block && pa.kn) gqa_mixed_kernel<true, true, NZ><<<grid, kPfWaves * 64, 0, s>>>(a, pa, npf);
@@ -3562,7 +3570,6 @@ extern "C" int aia_paged_attention_gqa(
     pa.batch = batch; pa.tokens = num_tokens;
     pa.scale_log2 = a.scale_log2;
     pa.out = a.out; pa.o_ts = a.o_ts; pa.o_hs = a.o_hs;
-    pa.units = reinterpret_cast<const int4*>(ws + L.pf);
     pa.dealt = reinterpret_cast<const int4*>(ws + L.pfw);
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);
@@ -3642,7 +3649,6 @@ extern "C" int aia_paged_attention_mla(
     pa.batch = batch; pa.tokens = num_tokens;
     pa.scale_log2 = a.scale_log2;
     pa.out = a.out; pa.o_ts = a.o_ts; pa.o_hs = a.o_hs;
-    pa.units = reinterpret_cast<const int4*>(ws + L.pf);
     pa.dealt = reinterpret_cast<const int4*>(ws + L.pfw);
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);

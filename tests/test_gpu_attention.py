@@ -543,3 +543,47 @@ def test_few_long_requests_merge_in_eighths(hq, hkv, d, lqs, lks):
     err = (out.float().cpu() - oracle(step)).abs().max().item()
     print(f"max-abs err {err:.3e}", flush=True)
     assert err <= TOL, err
+
+
+@pytest.mark.parametrize("hq,hkv,d,lqs", [
+    (32, 1, 64, [3, 1400, 90, 611]),       # one head over 8 XCDs, a decode-sized request beside
+    (64, 2, 64, [700, 20, 331]),           # 4 XCDs per head
+    (32, 4, 128, [1290, 37, 801]),         # 2 per head, one grid
+    (32, 4, 128, [1290, 2, 801]),          # ... with a split-K range
+    (24, 3, 128, [1500, 1024, 333]),       # heads that do not divide the XCDs
+    (64, 16, 64, [800, 450]),              # 2 heads per XCD
+    (14, 2, 64, [1100, 64, 705]),          # fits a round: long items cut
+])
+def test_ragged_prompts_dealt_largest_first(hq, hkv, d, lqs):
+    """Prompts of mixed lengths: past one round (512 work-groups) every
+    work-group has a record, each (unit, kv head) once, and ids come largest
+    first (within one of the 64 size buckets); within a round long items are
+    cut.  The output against the oracle."""
+    step = workloads.make_gqa_step(lqs=lqs, lks=lqs, num_q_heads=hq, num_kv_heads=hkv,
+                                   head_dim=d, block_size=16, seed=7)
+    plan = ops.AttentionPlan.from_lists(step.block_table.to(DEV), step.cu_seqlens_q,
+                                        step.seqlens_kv, hq, hkv, d, 16)
+    out = ops.paged_attention_gqa(step.q.to(DEV), step.k_cache.to(DEV), step.v_cache.to(DEV),
+                                  plan, step.scale)
+    err = (out.float().cpu() - oracle(step)).abs().max().item()
+    assert err <= TOL, err
+    L = ops.workspace_layout(len(lqs), sum(lqs), hq, hkv, d)
+    ws = plan.workspace.cpu()
+    hdr = ws[:64].view(torch.int32).tolist()
+    units, jobs = hdr[6], hdr[6] * hkv
+    items = sum(-(-lq * hq // hkv // 128) for lq in lqs if lq * hq // hkv >= 128)
+    assert hdr[8] == 0 and hdr[9] == jobs
+    rec = ws[L["pfw"]:L["pfw"] + 48 * jobs].view(torch.int32).view(jobs, 12)
+    assert len({(r[8], r[9]) for r in rec.tolist()}) == jobs
+    assert 0 <= rec[:, 8].min() and rec[:, 8].max() < units and rec[:, 9].max() < hkv
+    if items * hkv <= 512:
+        assert items < units and jobs <= 512
+    else:
+        assert units == items
+        size = (rec[:, 3] - rec[:, 2]).tolist()
+        bucket = -(-(max(size) + 1) // 64)
+        # a row of ids (one rank of every head) may straddle sizes only
+        # between heads' neighbouring ranks
+        span = max(8, hkv)
+        assert all(min(size[i:i + span]) + bucket >= max(size[i + span:], default=0)
+                   for i in range(0, jobs, span))

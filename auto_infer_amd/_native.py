@@ -126,4 +126,6 @@ def address(name):
 
 
 def call(name, *args):
-    check(getattr(load(), name)(*args), name)
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != AIA_OK:
+        check(rc, name)

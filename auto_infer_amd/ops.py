@@ -15,7 +15,15 @@ _BF16 = torch.bfloat16
 
 # Pointers and streams go to the C-ABI as plain ints: every pointer
 # parameter is declared c_void_p, which converts them (and None -> NULL).
+# The checks raise behind their conditions (a message formatted on every call
+# cost 0.1 - 0.4 us), and the stream's handle comes without a Stream object
+# (0.1 us against 1.8; the public call where that one is absent).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device):
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -29,19 +37,23 @@ def _require(cond, msg):
 
 
 def _check_device_tensor(t, name, dtype=None):
-    _require(isinstance(t, torch.Tensor), f"{name} must be a tensor")
-    _require(t.is_cuda, f"{name} must be on the GPU (no CPU fallback)")
-    if dtype is not None:
-        _require(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
+    if not isinstance(t, torch.Tensor):
+        raise ValueError(f"{name} must be a tensor")
+    if not t.is_cuda:
+        raise ValueError(f"{name} must be on the GPU (no CPU fallback)")
+    if dtype is not None and t.dtype != dtype:
+        raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
 
 
 def _row_stride(t, name):
     """Token stride of a (T, heads, dim) tensor whose (heads, dim) part is
     one contiguous row."""
-    _require(t.dim() == 3, f"{name} must be (tokens, heads, dim)")
-    _require(t.stride(2) == 1 and t.stride(1) == t.shape[2],
-             f"{name} rows (heads, dim) must be contiguous")
-    return t.stride(0)
+    if t.dim() != 3:
+        raise ValueError(f"{name} must be (tokens, heads, dim)")
+    s0, s1, s2 = t.stride()
+    if s2 != 1 or s1 != t.shape[2]:
+        raise ValueError(f"{name} rows (heads, dim) must be contiguous")
+    return s0
 
 
 # ---------------------------------------------------------------- KV write
@@ -64,18 +76,19 @@ def qk_norm_rope(qkv, num_q_heads, num_kv_heads, cos, sin, q_norm_weight=None,
     D = int(head_dim)
     if D not in (128, 64):
         raise NotImplementedError(f"qk_norm_rope: head_dim {D} (128 or 64)")
-    _require(width == (num_q_heads + 2 * num_kv_heads) * D,
-             f"qkv width {width} != (Hq + 2 Hkv) x {D}")
+    if width != (num_q_heads + 2 * num_kv_heads) * D:
+        raise ValueError(f"qkv width {width} != (Hq + 2 Hkv) x {D}")
     cs = []
     for t, name in ((cos, "cos"), (sin, "sin")):
         _check_device_tensor(t, name, _BF16)
-        _require(t.shape[0] == T and t.shape[-1] == D and t.numel() == T * D and t.stride(-1) == 1,
-                 f"{name} must hold one {D}-wide row per token")
+        if not (t.shape[0] == T and t.shape[-1] == D and t.numel() == T * D and t.stride(-1) == 1):
+            raise ValueError(f"{name} must hold one {D}-wide row per token")
         cs.append(t.stride(0))
     for t, name in ((q_norm_weight, "q_norm_weight"), (k_norm_weight, "k_norm_weight")):
         if t is not None:
             _check_device_tensor(t, name, _BF16)
-            _require(t.numel() == D and t.is_contiguous(), f"{name} must be {D} contiguous values")
+            if t.numel() != D or not t.is_contiguous():
+                raise ValueError(f"{name} must be {D} contiguous values")
     _native.call("aia_qk_norm_rope", _ptr(qkv), qkv.stride(0), T, num_q_heads, num_kv_heads, D,
                  _ptr(cos), cs[0], _ptr(sin), cs[1], _ptr(q_norm_weight), _ptr(k_norm_weight),
                  float(eps), _stream(qkv.device))
@@ -85,8 +98,9 @@ def qk_norm_rope(qkv, num_q_heads, num_kv_heads, cos, sin, q_norm_weight=None,
 
 def _rope_rows(t, name, T, width):
     _check_device_tensor(t, name, _BF16)
-    _require(t.shape[0] == T and t.shape[-1] == width and t.numel() == T * width and
-             t.stride(-1) == 1, f"{name} must hold one {width}-wide row per token")
+    if not (t.shape[0] == T and t.shape[-1] == width and t.numel() == T * width and
+            t.stride(-1) == 1):
+        raise ValueError(f"{name} must hold one {width}-wide row per token")
     return t.stride(0)
 
 
@@ -355,13 +369,15 @@ class AttentionPlan:
         """Re-run the device planner on the (possibly updated in place)
         metadata tensors; graph-capturable.  The plan is then valid on the
         current stream (attention calls on another stream wait for it)."""
-        self.stream = torch.cuda.current_stream(self.block_table.device)
+        device = self.block_table.device
+        self.stream = torch.cuda.current_stream(device)
+        self._on = (device, self.stream.cuda_stream)
         self._use_on(self.stream)
         _native.call("aia_attn_plan", _ptr(self.cu_seqlens_q), _ptr(self.seqlens_kv),
                      _ptr(self.block_table), self.block_table.stride(0), self.block_size,
                      self.batch, self.num_tokens, self.num_q_heads, self.num_kv_heads,
                      self.head_dim_v, self.num_waves, _ptr(self.workspace),
-                     self.workspace.numel(), _stream(self.block_table.device))
+                     self.workspace.numel(), self._on[1])
 
     def _use_on(self, stream):
         if stream not in self._streams:
@@ -413,7 +429,11 @@ def _ready(plan, device):
     """Order the attention launch after the planner: on another stream, make
     the current stream wait for the plan's stream (not allowed while
     capturing a graph, where the plan must be made on the capturing stream)
-    and record the plan's buffers as in use there."""
+    and record the plan's buffers as in use there.  Returns the current
+    stream's handle."""
+    raw = _stream(device)
+    if plan._on == (device, raw):
+        return raw
     cur = torch.cuda.current_stream(device)
     if cur != plan.stream:
         if torch.cuda.is_current_stream_capturing():
@@ -421,19 +441,22 @@ def _ready(plan, device):
                              "captured; call plan.replan() on the capturing stream")
         cur.wait_stream(plan.stream)
         plan._use_on(cur)
+    return raw
 
 
 def _check_out(out, name, shape, device):
     """A caller-supplied output: bf16 on the same GPU, of ``shape``, unit
     inner stride, rows (heads, dim) not overlapping."""
     _check_device_tensor(out, name, _BF16)
-    _require(out.device == device, f"{name} must be on {device}")
-    _require(tuple(out.shape) == tuple(shape), f"{name} must have shape {tuple(shape)}, "
-             f"got {tuple(out.shape)}")
-    _require(out.stride(-1) == 1, f"{name} must have unit inner stride")
-    if out.dim() == 3:
-        _require(out.stride(1) >= out.shape[2] and out.stride(0) >= out.shape[1] * out.stride(1),
-                 f"{name} rows must not overlap")
+    if out.device != device:
+        raise ValueError(f"{name} must be on {device}")
+    if out.shape != shape:
+        raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(out.shape)}")
+    st = out.stride()
+    if st[-1] != 1:
+        raise ValueError(f"{name} must have unit inner stride")
+    if len(st) == 3 and not (st[1] >= shape[2] and st[0] >= shape[1] * st[1]):
+        raise ValueError(f"{name} rows must not overlap")
 
 
 def paged_attention_gqa(query, key_cache, value_cache, plan, scale, out=None, flags=0,
@@ -449,38 +472,46 @@ def paged_attention_gqa(query, key_cache, value_cache, plan, scale, out=None, fl
     graph mode (see ``write_kv_nz``); results are the same as for the same
     values in the standard layout.
     """
-    _require(kv_layout in KV_LAYOUTS, f"kv_layout must be one of {sorted(KV_LAYOUTS)}")
+    if kv_layout not in KV_LAYOUTS:
+        raise ValueError(f"kv_layout must be one of {sorted(KV_LAYOUTS)}")
     flags |= KV_LAYOUTS[kv_layout]
     _check_device_tensor(query, "query", _BF16)
     _check_device_tensor(key_cache, "key_cache", _BF16)
     _check_device_tensor(value_cache, "value_cache", _BF16)
     _require(query.dim() == 3 and query.stride(2) == 1, "query must be (T, Hq, D), D contiguous")
-    T, hq, d = query.shape
+    shape = query.shape
+    T, hq, d = shape
     _require(key_cache.dim() == 4 and key_cache.is_contiguous() and value_cache.is_contiguous(),
              "caches must be contiguous (num_blocks, block_size, Hkv, D)")
-    nb, bs, hkv, dk = key_cache.shape
-    _require(tuple(value_cache.shape) == (nb, bs, hkv, dk), "value cache shape differs from key cache")
+    cshape = key_cache.shape
+    nb, bs, hkv, dk = cshape
+    _require(value_cache.shape == cshape, "value cache shape differs from key cache")
     _require(dk == d, "query head_dim differs from the cache's")
     _require(hq == plan.num_q_heads and hkv == plan.num_kv_heads and T == plan.num_tokens
              and bs == plan.block_size, "plan was made for another shape")
+    device = query.device
     if out is None:
-        out = torch.empty(T, hq, d, dtype=_BF16, device=query.device)
+        out = torch.empty(shape, dtype=_BF16, device=device)
     else:
-        _check_out(out, "out", (T, hq, d), query.device)
+        _check_out(out, "out", shape, device)
     kn_ts = vn_ts = 0
     if key_new is not None or value_new is not None:
         _check_device_tensor(key_new, "key_new", _BF16)
         _check_device_tensor(value_new, "value_new", _BF16)
-        _require(tuple(key_new.shape) == (T, hkv, d) and tuple(value_new.shape) == (T, hkv, d),
+        rows = (T, hkv, d)
+        _require(key_new.shape == rows and value_new.shape == rows,
                  "new K/V rows must be (tokens, Hkv, D)")
         kn_ts, vn_ts = _row_stride(key_new, "key_new"), _row_stride(value_new, "value_new")
-    _ready(plan, query.device)
-    _native.call("aia_paged_attention_gqa", _ptr(query), query.stride(0), query.stride(1),
-                 _ptr(key_cache), _ptr(value_cache), _ptr(plan.block_table),
-                 plan.block_table.stride(0), _ptr(plan.cu_seqlens_q), _ptr(plan.seqlens_kv),
-                 plan.batch, T, hq, hkv, d, bs, nb, float(scale), _ptr(out), out.stride(0),
-                 out.stride(1), _ptr(key_new), _ptr(value_new), kn_ts, vn_ts, plan.num_waves,
-                 flags, _ptr(plan.workspace), plan.workspace.numel(), _stream(query.device))
+    stream = _ready(plan, device)
+    q_ts, q_hs, _ = query.stride()
+    o_ts, o_hs, _ = out.stride()
+    table, ws = plan.block_table, plan.workspace
+    _native.call("aia_paged_attention_gqa", query.data_ptr(), q_ts, q_hs,
+                 key_cache.data_ptr(), value_cache.data_ptr(), table.data_ptr(),
+                 table.stride(0), plan.cu_seqlens_q.data_ptr(), plan.seqlens_kv.data_ptr(),
+                 plan.batch, T, hq, hkv, d, bs, nb, float(scale), out.data_ptr(), o_ts,
+                 o_hs, _ptr(key_new), _ptr(value_new), kn_ts, vn_ts, plan.num_waves,
+                 flags, ws.data_ptr(), ws.numel(), stream)
     return out
 
 
@@ -513,11 +544,11 @@ def paged_attention_mla(q_latent, latent_cache, plan, scale, out=None, flags=0):
         out = torch.empty(T, h, MLA_LATENT, dtype=_BF16, device=q_latent.device)
     else:
         _check_out(out, "out", (T, h, MLA_LATENT), q_latent.device)
-    _ready(plan, q_latent.device)
+    stream = _ready(plan, q_latent.device)
     _native.call("aia_paged_attention_mla", _ptr(q_latent), q_latent.stride(0),
                  q_latent.stride(1), _ptr(latent_cache), _ptr(plan.block_table),
                  plan.block_table.stride(0), _ptr(plan.cu_seqlens_q), _ptr(plan.seqlens_kv),
                  plan.batch, T, h, MLA_LATENT, MLA_ROPE, bs, nb, float(scale), _ptr(out),
                  out.stride(0), out.stride(1), plan.num_waves, flags, _ptr(plan.workspace),
-                 plan.workspace.numel(), _stream(q_latent.device))
+                 plan.workspace.numel(), stream)
     return out

@@ -129,6 +129,9 @@ constexpr int kPfKeys = AIA_PF_KEYS;         // keys per staged K/V tile (32 or 
 #endif
 constexpr int kPfTargetWgs = AIA_PF_TARGET;
 constexpr int kPfCutSlots = 512;     // most work-groups (units x kv heads) of a step with cut items
+constexpr int kPfRecBytes = 48;      // a dealt work-group's record: three int4
+static_assert(2 * kPfTargetWgs >= kPfCutSlots && (2 * kPfTargetWgs - kPfCutSlots) * kPfRows * 8 >=
+              kPfCutSlots * kPfRecBytes, "partials and records of a step with cut items");
 #ifndef AIA_MLA_LPT
 #define AIA_MLA_LPT 1
 #endif
@@ -247,28 +250,27 @@ Layout layout(int32_t batch, int32_t tokens, const Geometry& g, int32_t dv, int3
   const int64_t pf_reqs = pf_rows / kPfRows < batch ? pf_rows / kPfRows : batch;
   L.pf_cap = (pf_rows + kPfRows - 1) / kPfRows + pf_reqs;
   // Items are cut only while their units x kv heads stay within kPfTargetWgs
-  // or two work-groups per CU (512), and a cut item has two units or more.
-  // So partials fill at most kPfCutSlots row blocks, and the records of
-  // work-groups past kPfTargetWgs lie behind those (they add to the workspace
-  // only past about 100,000 work-groups).
-  static_assert(2 * kPfTargetWgs >= kPfCutSlots, "row blocks of all partials");
+  // or two work-groups per CU (512), so the partials of a step with cut items
+  // fill at most kPfCutSlots row blocks.  The records of the dealt
+  // work-groups follow the (max, sum) pairs of those blocks: a step within
+  // kPfCutSlots work-groups ends in front of the partial values, and the
+  // records of a larger one, which cuts nothing and has no partials, run on
+  // through them (they add to the workspace only past 300,000 work-groups).
   const int64_t split_units = g.pf ? 2 * ((kPfTargetWgs + g.hkv - 1) / g.hkv) + 1 : 0;
   L.pf_unit_cap = L.pf_cap > split_units ? L.pf_cap : split_units;
   L.pf_mrg_cap = g.pf ? (kPfTargetWgs + g.hkv - 1) / g.hkv : 0;
   L.pf_slots = split_units * g.hkv;             // partial row blocks
   L.pf = off;       off = align256(off + L.pf_unit_cap * 32);              // two int4 per unit
   L.pfm = off;      off = align256(off + L.pf_mrg_cap * 16);
-  L.pfw = off;      off = align256(off + (g.pf ? kPfTargetWgs * 48 : 0));   // dealt work-groups
-  L.pf_ml = off;    off = align256(off + L.pf_slots * kPfRows * 8);
+  L.pf_ml = off;
+  L.pfw = off + (g.pf ? kPfCutSlots * kPfRows * 8 : 0);
+  off = align256(off + L.pf_slots * kPfRows * 8 + (g.pf ? kPfTargetWgs * kPfRecBytes : 0));
   L.pf_o = off;
-  const int64_t row_block = kPfRows * (int64_t)dv * 2, more = L.pf_unit_cap * g.hkv - kPfTargetWgs;
-  const int64_t with_records = more > 0 ? kPfCutSlots * row_block + more * 48 : 0;
-  off = align256(off + max(L.pf_slots * row_block, with_records));
-  L.total = off;
+  off += L.pf_slots * kPfRows * (int64_t)dv * 2;
+  if (g.pf) off = std::max(off, L.pfw + L.pf_unit_cap * g.hkv * kPfRecBytes);
+  L.total = align256(off);
   return L;
 }
-// Offset of the work-group records past kPfTargetWgs.
-int64_t more_records(const Layout& L, int32_t dv) { return L.pf_o + kPfCutSlots * kPfRows * (int64_t)dv * 2; }
 
 // Number of key ranges (= work-groups).  Default: about kDefaultWaves waves
 // in flight for GQA (one per kv head of a group), three four-wave groups per
@@ -393,7 +395,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     int32_t* __restrict__ hdr, int32_t* __restrict__ seg, int32_t* __restrict__ wave_rec,
     int32_t* __restrict__ req_scratch,
     int32_t* __restrict__ mrg, int4* __restrict__ pf_units, int4* __restrict__ pf_mrg,
-    int4* __restrict__ pf_wg, int4* __restrict__ pf_wg_more, int32_t pf_cap, int32_t pf_unit_cap, int32_t pf_mrg_cap,
+    int4* __restrict__ pf_wg, int32_t pf_cap, int32_t pf_unit_cap, int32_t pf_mrg_cap,
     int32_t seg_cap, int32_t fix_cap) {
   __shared__ __attribute__((aligned(16))) int lds[kPlanLds];
   __shared__ int wave_sums[kPlanThreads / 64];
@@ -577,7 +579,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     pmerges = mcarry2;
     if (units > pf_unit_cap || pmerges > pf_mrg_cap) { units = 0; pmerges = 0; overflow = 1; }
 
-    // 1c) Work-group b's record at pf_wg[b] (pf_wg_more past kPfTargetWgs): its unit record (two int4),
+    // 1c) Work-group b's record at pf_wg[3 b]: its unit record (two int4),
     // then {unit, kv head}, so a work-group loads it beside the header
     // instead of after it; hdr[9] = the number written.  Work-groups go to
     // the XCDs round-robin by id, so b takes XCD b % 8.
@@ -600,9 +602,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     //   XCD gets a contiguous run of (kv head, unit) pairs, kv-head major.
     // Absorbed-MLA units run one per CU and are always dealt largest first.
     const int jobs = units * g.hkv;
-    auto wg_record = [&](int id) {
-      return id < kPfTargetWgs ? pf_wg + 3 * id : pf_wg_more + 3 * (id - kPfTargetWgs);
-    };
     const bool lpt = (dv == 512 && AIA_MLA_LPT) || jobs > 2 * g.ncu;
     const bool pair_deal = !lpt && alone && jobs > g.ncu && jobs <= 2 * g.ncu;
     if (!pair_deal && !lpt) {
@@ -612,7 +611,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         const int x = id % kXcdsPlan, i = id / kXcdsPlan;
         const int pair = x * q + min(x, r) + i;          // the run of XCD id % 8
         const int kvh = pair / units, u = pair - kvh * units;
-        int4* rec = wg_record(id);
+        int4* rec = pf_wg + 3 * (int64_t)id;
         rec[0] = pf_units[2 * u];
         rec[1] = pf_units[2 * u + 1];
         rec[2] = make_int4(u, kvh, 0, 0);
@@ -642,7 +641,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         const int4 e = pf_units[2 * u], e2 = pf_units[2 * u + 1];
         const int r = atomicAdd(&pf_hist[bucket(e.w - e.z)], 1);
         auto put = [&](int id, int kvh) {
-          int4* rec = wg_record(id);
+          int4* rec = pf_wg + 3 * (int64_t)id;
           rec[0] = e;
           rec[1] = e2;
           rec[2] = make_int4(u, kvh, 0, 0);
@@ -1657,16 +1656,11 @@ struct PrefillArgs {
   const int4* dealt;         // work-group b: {request, first row, first tile, end tile},
                              // {first query token, query tokens, keys, first tile's block id},
                              // {unit, kv head}
-  const int4* dealt_more;    // ... of work-group kPfTargetWgs + b
   const int32_t* hdr;
   uint16_t* part_o;          // partial row blocks of chunked items (fp16, scaled per row)
   float2* part_ml;
   int32_t part_units;        // units the partial buffer holds
 };
-
-__device__ __forceinline__ const int4* wg_record(const PrefillArgs& a, int wg) {
-  return wg < kPfTargetWgs ? a.dealt + 3 * wg : a.dealt_more + 3 * (wg - kPfTargetWgs);
-}
 
 // LDS rows of the staged K and V tiles are 2 D bytes, unpadded: the direct
 // loads write whole 1 KB runs, so the chunks of each row are swizzled
@@ -1717,7 +1711,7 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
   constexpr int RC = D / 8;         // 16-byte chunks per K / V row
   // The planner writes work-group b's record at dealt[b] (the grid is as long
   // as the list can be); it is loaded beside the header rather than after it.
-  const int4* rec = wg_record(a, wg);
+  const int4* rec = a.dealt + 3 * (int64_t)wg;
   const int4 it = rec[0], iq = rec[1], uk = rec[2];
   const int count = a.hdr[6];
   if (wg >= count * a.hkv) return;
@@ -2930,7 +2924,7 @@ void mla_prefill_kernel(PrefillArgs a) {
   __shared__ int rerun_flag;
   const int wg = blockIdx.x;
   // this work-group's unit, as the GQA units take theirs (one kv head)
-  const int4* rec = wg_record(a, wg);
+  const int4* rec = a.dealt + 3 * (int64_t)wg;
   const int4 it = rec[0], iq = rec[1];
   const int unit = rec[2].x;
   const int count = a.hdr[6];
@@ -3506,7 +3500,6 @@ extern "C" int aia_attn_plan(const int32_t* cu_seqlens_q, const int32_t* seqlens
       reinterpret_cast<int32_t*>(ws + L.req),
       reinterpret_cast<int32_t*>(ws + L.mrg), reinterpret_cast<int4*>(ws + L.pf),
       reinterpret_cast<int4*>(ws + L.pfm), reinterpret_cast<int4*>(ws + L.pfw),
-      reinterpret_cast<int4*>(ws + more_records(L, head_dim_v)),
       (int32_t)L.pf_cap, (int32_t)L.pf_unit_cap,
       (int32_t)L.pf_mrg_cap, (int32_t)L.seg_cap,
       small_geometry(g, head_dim_v, batch, L.seg_cap) ? (int32_t)L.part_cap : 0);
@@ -3593,7 +3586,6 @@ extern "C" int aia_paged_attention_gqa(
     pa.scale_log2 = a.scale_log2;
     pa.out = a.out; pa.o_ts = a.o_ts; pa.o_hs = a.o_hs;
     pa.dealt = reinterpret_cast<const int4*>(ws + L.pfw);
-    pa.dealt_more = reinterpret_cast<const int4*>(ws + more_records(L, head_dim));
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);
     pa.part_ml = reinterpret_cast<float2*>(ws + L.pf_ml);
@@ -3673,7 +3665,6 @@ extern "C" int aia_paged_attention_mla(
     pa.scale_log2 = a.scale_log2;
     pa.out = a.out; pa.o_ts = a.o_ts; pa.o_hs = a.o_hs;
     pa.dealt = reinterpret_cast<const int4*>(ws + L.pfw);
-    pa.dealt_more = reinterpret_cast<const int4*>(ws + more_records(L, kMlaV));
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);
     pa.part_ml = reinterpret_cast<float2*>(ws + L.pf_ml);

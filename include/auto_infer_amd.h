@@ -78,8 +78,11 @@ int aia_attn_workspace_bytes(int32_t batch, int32_t num_tokens,
  * lists themselves).  Writes up to `count` int64 values, -1 past the end:
  * byte offsets of the header, segment records, range records, split
  * partials (max/sum, values), request offsets, merge records, prefill unit
- * records, prefill merge records, dealt prefill work-groups, prefill
- * partials (max/sum, values) and the total size; then the capacities
+ * records, prefill merge records, dealt prefill work-groups (header word 9
+ * counts them, 48 bytes each; they lie between the prefill partials' max/sum
+ * pairs and values, and a step of more than 512, which has no partials, fills
+ * the values' place too), prefill partials (max/sum, values) and the total
+ * size; then the capacities
  * (segments, merge records, prefill items, prefill units, prefill merges),
  * the range count, and the prefill item rows and tile keys. */
 int aia_attn_workspace_layout(int32_t batch, int32_t num_tokens, int32_t num_q_heads,

@@ -573,10 +573,7 @@ def test_ragged_prompts_dealt_largest_first(hq, hkv, d, lqs):
     units, jobs = hdr[6], hdr[6] * hkv
     items = sum(-(-lq * hq // hkv // 128) for lq in lqs if lq * hq // hkv >= 128)
     assert hdr[8] == 0 and hdr[9] == jobs
-    # 448 records, the rest behind the 512 row blocks that partials may fill
-    more = L["pf_o"] + 512 * 128 * d * 2
-    rec = torch.cat([ws[L["pfw"]:L["pfw"] + 48 * min(jobs, 448)],
-                     ws[more:more + 48 * max(0, jobs - 448)]]).view(torch.int32).view(jobs, 12)
+    rec = ws[L["pfw"]:L["pfw"] + 48 * jobs].view(torch.int32).view(jobs, 12)
     assert len({(r[8], r[9]) for r in rec.tolist()}) == jobs
     assert 0 <= rec[:, 8].min() and rec[:, 8].max() < units and rec[:, 9].max() < hkv
     if items * hkv <= 512:

@@ -53,6 +53,24 @@ def test_workspace_query():
     assert out.value < 64 << 20 < big.value
 
 
+@pytest.mark.parametrize("hkv,group,d", [(1, 16, 512), (1, 7, 64), (2, 7, 64), (3, 8, 128),
+                                         (4, 7, 128), (8, 8, 128), (300, 1, 128)])
+@pytest.mark.parametrize("tokens", [256, 2048, 16384, 1 << 21])
+def test_every_prefill_work_group_has_a_record_in_the_layout(hkv, group, d, tokens):
+    """aia_attn_workspace_layout's one offset of the dealt work-groups holds
+    a record (48 bytes) for every one a step can have: behind the (max, sum)
+    pairs of the 512 row blocks that cut items may fill, those of a step with
+    cut items (at most 512) in front of the partial values, all inside the
+    workspace."""
+    from auto_infer_amd import ops
+    L = ops.workspace_layout(1, tokens, hkv * group, hkv, d)
+    assert L["pf_unit_cap"] * hkv >= -(-tokens * group // 128) * hkv
+    assert L["pfw"] >= L["pf_ml"] + 512 * 128 * 8
+    assert L["pfw"] + 48 * 512 <= L["pf_o"]
+    assert L["pfw"] + 48 * L["pf_unit_cap"] * hkv <= L["total"]
+    assert L["pf_o"] + 512 * 128 * d * 2 <= L["total"]
+
+
 def test_argument_validation_of_the_fused_kernels_without_gpu():
     """Bad arguments are rejected before any device call, with the mapped
     exception types."""

@@ -250,8 +250,10 @@ Layout layout(int32_t batch, int32_t tokens, const Geometry& g, int32_t dv, int3
   const int64_t pf_reqs = pf_rows / kPfRows < batch ? pf_rows / kPfRows : batch;
   L.pf_cap = (pf_rows + kPfRows - 1) / kPfRows + pf_reqs;
   // Items are cut only while their units x kv heads stay within kPfTargetWgs
-  // or two work-groups per CU (512), so the partials of a step with cut items
-  // fill at most kPfCutSlots row blocks.  The records of the dealt
+  // or two work-groups per CU (512), so the (max, sum) pairs of a step with
+  // cut items fill at most kPfCutSlots row blocks; the units with partials,
+  // kPfTargetWgs / Hkv of them at most, have a slot of two fp16 row blocks,
+  // which those with fp32 partials fill.  The records of the dealt
   // work-groups follow the (max, sum) pairs of those blocks: a step within
   // kPfCutSlots work-groups ends in front of the partial values, and the
   // records of a larger one, which cuts nothing and has no partials, run on
@@ -452,6 +454,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // Every loop below runs over the flat item list (request-major, each
   // request's items last rows first), one item per thread.
   int units = 0, pmerges = 0, dealt = 0;
+  int nwide = 0;            // units with fp32 partials
   // Fill target.  Absorbed-MLA units (158 KB of LDS) run one per CU: few
   // items are cut into one round of units (8 x 64 tokens at 4096 keys: 172
   // us against 205 at 448), many into about 1.75 rounds so the causal
@@ -478,19 +481,24 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       return (kend + kPfKeys - 1) / kPfKeys;
     };
     int chunk = 0x7fffffff, wtot = 0;
-    // the least chunk above `lo` and up to `hi` whose units number at most ucap
-    auto least_chunk = [&](int lo, int hi, int ucap) {
+    int fill = 0;             // wide: the chunk that fills the chip
+    bool wide = false;        // items of up to `fill` tiles are cut too
+    // the least chunk above `lo` and up to `hi` whose units number at most
+    // ucap, those of cut items at most ccap
+    auto least_chunk = [&](int lo, int hi, int ucap, int ccap) {
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        int nu = 0;
+        int nu = 0, nc = 0;
         for (int f = tid; f < pcarry; f += kPlanThreads) {
           int b, r0;
           const int nt = item_at(f, b, r0);
-          nu += nt > mid ? (nt + mid - 1) / mid : 1;
+          const int k = nt > mid ? (nt + mid - 1) / mid : 1;
+          nu += k;
+          nc += k > 1 ? k : 0;
         }
-        int utot;
-        block_exclusive_scan(nu, wave_sums, &utot);
-        if (utot <= ucap) hi = mid; else lo = mid + 1;
+        int2 tot2;
+        block_exclusive_scan2(make_int2(nu, nc), wave_sums2, &tot2);
+        if (tot2.x <= ucap && tot2.y <= ccap) hi = mid; else lo = mid + 1;
       }
       return hi;
     };
@@ -520,25 +528,35 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       // keeps units x kv heads within the target: one round of work-groups
       const int64_t room = pf_target - (int64_t)pcarry * g.hkv;
       chunk = max(kPfMinChunk, (int)(((int64_t)wtot * g.hkv + room - 1) / room));
-      // That bound is loose.  Alone on the chip, the least chunk whose units
-      // still fit evens the work-groups out (the slowest one sets the kernel
-      // time), found by a binary search, one block reduction per probe.
-      // Beside split-K ranges the loose bound stays: its fewer work-groups
-      // leave slots for the HBM-bound ranges.
+      // That bound is loose.  In a step with no split-K segments the least
+      // chunk whose units still fit evens the work-groups out (the slowest
+      // one sets the kernel time), found by a binary search, one block
+      // reduction per probe.  Beside split-K ranges the loose bound stays:
+      // its fewer work-groups leave slots for the HBM-bound ranges.
       const int ucap = pf_target / g.hkv;
-      if (alone) chunk = least_chunk(max(kPfMinChunk, (wtot + ucap - 1) / ucap), chunk, ucap);
+      if (carry == 0)
+        chunk = least_chunk(max(kPfMinChunk, (wtot + ucap - 1) / ucap), chunk, ucap, ucap);
     }
     // Ragged prompts: items that nearly fill the target are left (almost)
     // uncut by it, and the longest sets the kernel time.  They are cut for
     // two work-groups per CU where that shortens the longest by an eighth (7
     // prompts of 40 to 1657 tokens, 14 / 2 heads of 64: 37.0 us per call to
-    // 30.5; 4 chunks of 512 tokens at 4096 keys, whose items are all long,
+    // 31.8; 4 chunks of 512 tokens at 4096 keys, whose items are all long,
     // 126 uncut and 130 cut; 768 or more work-groups 3 - 10 us slower on
-    // either).
+    // either).  Items that fill the chip without this cut keep their sums in
+    // fp32: the list then starts with the units of those items (hdr[11] of
+    // them), whose partials are fp32 values, then come those of the items that
+    // are cut for the fill too, then the whole ones, so that only cut items'
+    // units have partial slots.
     if (even) {
       const int ucap = pair_slots / g.hkv, top = min(longest, chunk);
-      const int c2 = least_chunk(min(top, max(kPfMinChunk, (wtot + ucap - 1) / ucap)), top, ucap);
-      if (8 * c2 <= 7 * top) chunk = c2;
+      const int c2 = least_chunk(min(top, max(kPfMinChunk, (wtot + ucap - 1) / ucap)), top, ucap,
+                                 min(ucap, pf_mrg_cap));
+      if (8 * c2 <= 7 * top) {
+        fill = chunk;
+        chunk = c2;
+        wide = true;
+      }
     }
     int ucarry = 0, mcarry2 = 0;
     for (int base = 0; base < pcarry; base += kPlanThreads) {
@@ -548,9 +566,19 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         nt = item_at(f, b, r0);
         k = nt > chunk ? (nt + chunk - 1) / chunk : 1;
       }
+      const int kc = k > 1 ? k : 0, kw = wide && nt <= fill ? kc : 0;   // units of a cut item, fp32
       int2 tot2;
-      const int2 ex2 = block_exclusive_scan2(make_int2(k, k > 1 ? 1 : 0), wave_sums2, &tot2);
-      const int u = ucarry + ex2.x, mm = mcarry2 + ex2.y;
+      // (units of cut items and their records stay below 1024; wide steps have
+      // at most 512 units)
+      const int2 ex2 = block_exclusive_scan2(make_int2(k | kw << 16, kc << 10 | (k > 1)), wave_sums2, &tot2);
+      const int mm = mcarry2 + (ex2.y & 1023);
+      int u = ucarry + ex2.x;
+      if (wide) {     // (fewer items than threads: one round lists them all)
+        const int w_before = ex2.x >> 16, c_before = ex2.y >> 10;
+        nwide = tot2.x >> 16;
+        tot2.x &= 0xffff;
+        u = kw ? w_before : kc ? nwide + c_before - w_before : (tot2.y >> 10) + (ex2.x & 0xffff) - c_before;
+      }
       if (f < pcarry && u + k <= pf_unit_cap && mm + (k > 1) <= pf_mrg_cap) {
         if (k > 1) {
           // {first query token, first row, first unit, units | item rows << 16}
@@ -573,7 +601,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         }
       }
       ucarry += tot2.x;
-      mcarry2 += tot2.y;
+      mcarry2 += tot2.y & 1023;
     }
     units = ucarry;
     pmerges = mcarry2;
@@ -913,6 +941,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     hdr[8] = overflow ? -1 : 0;   // status: -1 = the metadata asked for more work than fits
     hdr[9] = overflow ? 0 : dealt;
     hdr[10] = fixed ? 1 : 0;
+    hdr[11] = nwide;
     // sentinel record so readers may look one past the end
     int* r = seg + (int64_t)nseg * 8;
     r[0] = 0; r[1] = 0; r[2] = 0; r[3] = 0; r[4] = 0;
@@ -1657,7 +1686,7 @@ struct PrefillArgs {
                              // {first query token, query tokens, keys, first tile's block id},
                              // {unit, kv head}
   const int32_t* hdr;
-  uint16_t* part_o;          // partial row blocks of chunked items (fp16, scaled per row)
+  uint16_t* part_o;          // partials of chunked items, two fp16 row blocks per (unit, kv head)
   float2* part_ml;
   int32_t part_units;        // units the partial buffer holds
 };
@@ -1788,6 +1817,7 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
   // not cover them all writes a partial
   if (t0 < 0 || t1 < t0 || t1 > ntiles) return;
   const bool whole = t0 == 0 && t1 == ntiles;
+  const bool wide = unit < a.hdr[11];
   if (!whole && unit >= a.part_units) return;
 
   // Loader: thread tid moves 16-byte chunk (tid % RC) of keys kLdKeys i + tid / RC
@@ -2077,9 +2107,10 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
     // y = O / c in fp16, c = the row's largest |O| (1 for an all-zero row),
     // with (m + log2 c, l / c) in place of (m, l).  The merge's log-sum-exp
     // rule then folds c back exactly (its weights are exp2(m - M)), and the
-    // partials take half the bytes of fp32 ones.
+    // partials take half the bytes of fp32 ones.  The first hdr[11] units of
+    // the list keep O and (m, l) as they are, in fp32 (see the planner).
     float cmax = 0.f;
-    if (!whole) {
+    if (!whole && !wide) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -2087,10 +2118,18 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
       cmax = aia::group4_max(cmax);
     }
     if (!rv[rt]) continue;
+    if (!whole && wide) {
+      const int64_t prow = ((int64_t)unit * a.hkv + kvh) * kPfRows + (wid * kPfRt + rt) * kRows + n;
+      float* pp = reinterpret_cast<float*>(a.part_o) + prow * D;      // its block, whole
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<float4_t*>(pp + 16 * dt + 4 * g) = o[rt][dt];
+      if (g == 0) a.part_ml[prow] = make_float2(m[rt], lsum[rt]);
+      continue;
+    }
     if (!whole) {
       const float c = cmax > 0.f ? cmax : 1.f, ic = 1.f / c;
-      const int64_t prow = ((int64_t)unit * a.hkv + kvh) * kPfRows + (wid * kPfRt + rt) * kRows + n;
-      uint16_t* pp = a.part_o + prow * D;
+      const int64_t blk = (int64_t)unit * a.hkv + kvh, r = (wid * kPfRt + rt) * kRows + n;
+      uint16_t* pp = a.part_o + (2 * blk * kPfRows + r) * D;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         uint2 hv;
@@ -2098,7 +2137,7 @@ __device__ __forceinline__ void gqa_prefill_body(const PrefillArgs& a, int wg,
         hv.y = pack_f16x2(o[rt][dt][2] * ic, o[rt][dt][3] * ic);
         *reinterpret_cast<uint2*>(pp + 16 * dt + 4 * g) = hv;
       }
-      if (g == 0) a.part_ml[prow] = make_float2(m[rt] + __log2f(c), lsum[rt] * ic);
+      if (g == 0) a.part_ml[blk * kPfRows + r] = make_float2(m[rt] + __log2f(c), lsum[rt] * ic);
       continue;
     }
     const float inv = lsum[rt] > 0.f ? 1.f / lsum[rt] : 0.f;
@@ -2244,7 +2283,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   const int* hv = a.hdr + vz;
   const int4 m0_v = mp[0], m1_v = mp[1];
   const int4 pr_v = pp0[0];
-  const int h0 = hv[0], h2 = hv[2], h5 = hv[5], h7 = hv[7], h8 = hv[8], h10 = hv[10];
+  const int h0 = hv[0], h2 = hv[2], h5 = hv[5], h7 = hv[7], h8 = hv[8], h10 = hv[10], h11 = hv[11];
   auto fold_into = [](float& mx, float& ls, float4 (&acc)[kMergeDims / 4], float2 ml,
                       const float4 (&x)[kMergeDims / 4]) {
     const float mn = fmaxf(mx, ml.x);
@@ -2301,6 +2340,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   const int npm_hdr = __builtin_amdgcn_readfirstlane(h7);
   const int status = __builtin_amdgcn_readfirstlane(h8);   // planner status, used at the end
   const int npm = a.pf_mrg ? npm_hdr : 0;
+  const int nwide = __builtin_amdgcn_readfirstlane(h11);       // units with fp32 partials
   const int fixed_plan = FIXL > 0 ? __builtin_amdgcn_readfirstlane(h10) : 0;
   const int4 pr0 = make_int4(__builtin_amdgcn_readfirstlane(pr_v.x), __builtin_amdgcn_readfirstlane(pr_v.y),
                              __builtin_amdgcn_readfirstlane(pr_v.z), __builtin_amdgcn_readfirstlane(pr_v.w));
@@ -2467,9 +2507,9 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
   }
 
   // Prefill chunk merges, one work item per (record, kv head, pf_rpp rows):
-  // thread (row r, 8 dims) folds the record's fp16 partials (scaled per row,
-  // see the prefill kernel) with the same rule, 8 at a time so a batch costs
-  // one round trip.
+  // thread (row r, 8 dims) folds the record's partials (fp16 scaled per row,
+  // or fp32, see the prefill kernel) with the same rule, a batch at a time so it
+  // costs one round trip.
   const int64_t pitems = (int64_t)npm * per_rec;
   for (int64_t it = blockIdx.x; it < pitems; it += gridDim.x) {
     const int rec = (int)(it / per_rec);
@@ -2482,33 +2522,45 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
     if (rl >= rows) continue;
     float4 acc[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
     float mx = -1e30f, ls = 0.f;
-    for (int j0 = 0; j0 < k; j0 += 8) {
-      float2 ml[8];
-      float4 x[8][2];
+    auto fold_parts = [&](auto wide_tag) __attribute__((always_inline)) {
+      constexpr bool W = decltype(wide_tag)::value;
+      constexpr int B = W ? 4 : 8;       // parts whose loads go out together (same registers)
+      for (int j0 = 0; j0 < k; j0 += B) {
+        float2 ml[B];
+        float4 x[B][2];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (j0 + j >= k) break;                    // k is the same for the whole work-group
-        const int64_t prow = ((int64_t)(u0 + j0 + j) * a.hkv + kvh) * kPfRows + rl;
-        ml[j] = a.pf_ml[prow];
-        const uint4 h = *reinterpret_cast<const uint4*>(a.pf_o + prow * a.dv + c);
-        const half2_t h0 = __builtin_bit_cast(half2_t, h.x), h1 = __builtin_bit_cast(half2_t, h.y);
-        const half2_t h2 = __builtin_bit_cast(half2_t, h.z), h3 = __builtin_bit_cast(half2_t, h.w);
-        x[j][0] = make_float4((float)h0[0], (float)h0[1], (float)h1[0], (float)h1[1]);
-        x[j][1] = make_float4((float)h2[0], (float)h2[1], (float)h3[0], (float)h3[1]);
-      }
+        for (int j = 0; j < B; ++j) {
+          if (j0 + j >= k) break;                  // k is the same for the whole work-group
+          const int64_t blk = (int64_t)(u0 + j0 + j) * a.hkv + kvh;
+          ml[j] = a.pf_ml[blk * kPfRows + rl];
+          if (W) {
+            const float* f = reinterpret_cast<const float*>(a.pf_o) + (blk * kPfRows + rl) * a.dv + c;
+            x[j][0] = reinterpret_cast<const float4*>(f)[0];
+            x[j][1] = reinterpret_cast<const float4*>(f)[1];
+          } else {
+            const uint4 h = *reinterpret_cast<const uint4*>(a.pf_o + (2 * blk * kPfRows + rl) * a.dv + c);
+            const half2_t h0 = __builtin_bit_cast(half2_t, h.x), h1 = __builtin_bit_cast(half2_t, h.y);
+            const half2_t h2 = __builtin_bit_cast(half2_t, h.z), h3 = __builtin_bit_cast(half2_t, h.w);
+            x[j][0] = make_float4((float)h0[0], (float)h0[1], (float)h1[0], (float)h1[1]);
+            x[j][1] = make_float4((float)h2[0], (float)h2[1], (float)h3[0], (float)h3[1]);
+          }
+        }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (j0 + j >= k) break;
-        const float mn = fmaxf(mx, ml[j].x);
-        const float sa = __builtin_amdgcn_exp2f(mx - mn), sb = __builtin_amdgcn_exp2f(ml[j].x - mn);
-        ls = ls * sa + ml[j].y * sb;
-        acc[0].x = acc[0].x * sa + x[j][0].x * sb; acc[0].y = acc[0].y * sa + x[j][0].y * sb;
-        acc[0].z = acc[0].z * sa + x[j][0].z * sb; acc[0].w = acc[0].w * sa + x[j][0].w * sb;
-        acc[1].x = acc[1].x * sa + x[j][1].x * sb; acc[1].y = acc[1].y * sa + x[j][1].y * sb;
-        acc[1].z = acc[1].z * sa + x[j][1].z * sb; acc[1].w = acc[1].w * sa + x[j][1].w * sb;
-        mx = mn;
+        for (int j = 0; j < B; ++j) {
+          if (j0 + j >= k) break;
+          const float mn = fmaxf(mx, ml[j].x);
+          const float sa = __builtin_amdgcn_exp2f(mx - mn), sb = __builtin_amdgcn_exp2f(ml[j].x - mn);
+          ls = ls * sa + ml[j].y * sb;
+          acc[0].x = acc[0].x * sa + x[j][0].x * sb; acc[0].y = acc[0].y * sa + x[j][0].y * sb;
+          acc[0].z = acc[0].z * sa + x[j][0].z * sb; acc[0].w = acc[0].w * sa + x[j][0].w * sb;
+          acc[1].x = acc[1].x * sa + x[j][1].x * sb; acc[1].y = acc[1].y * sa + x[j][1].y * sb;
+          acc[1].z = acc[1].z * sa + x[j][1].z * sb; acc[1].w = acc[1].w * sa + x[j][1].w * sb;
+          mx = mn;
+        }
       }
-    }
+    };
+    if (__builtin_amdgcn_readfirstlane(u0) < nwide) fold_parts(std::true_type{});
+    else fold_parts(std::false_type{});
     const float inv = ls > 0.f ? 1.f / ls : 0.f;
     const int tok = row / a.group, head = kvh * a.group + (row - tok * a.group);
     uint16_t* op = a.out + (int64_t)(q_begin + tok) * a.o_ts + (int64_t)head * a.o_hs + c;
@@ -3288,7 +3340,7 @@ void mla_prefill_kernel(PrefillArgs a) {
       if (orow >= row_end) break;                     // uniform over the wave
       const uint4 x = *reinterpret_cast<const uint4*>(ob + (16 * wid + i) * kOutRow + 16 * lane);
       uint16_t* dst = whole ? a.out + (int64_t)(q_begin + orow / G) * a.o_ts + (int64_t)(orow % G) * a.o_hs
-                            : a.part_o + ((int64_t)unit * kPfRows + r) * kMlaV;
+                            : a.part_o + ((int64_t)2 * unit * kPfRows + r) * kMlaV;
       reinterpret_cast<uint4*>(dst)[lane] = x;
     }
   }
@@ -3589,7 +3641,7 @@ extern "C" int aia_paged_attention_gqa(
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);
     pa.part_ml = reinterpret_cast<float2*>(ws + L.pf_ml);
-    pa.part_units = kPfCutSlots / g.hkv;
+    pa.part_units = (int32_t)std::min<int64_t>(kPfCutSlots, L.pf_slots / 2) / g.hkv;
   }
   const bool one_block = block_size % kPfKeys == 0;
   if (int rc = (flags & AIA_ATTN_KV_NZ) ? launch_gqa<true>(a, pa, L, g, head_dim, waves, one_block, s)
@@ -3668,7 +3720,7 @@ extern "C" int aia_paged_attention_mla(
     pa.hdr = a.hdr;
     pa.part_o = reinterpret_cast<uint16_t*>(ws + L.pf_o);
     pa.part_ml = reinterpret_cast<float2*>(ws + L.pf_ml);
-    pa.part_units = kPfCutSlots;
+    pa.part_units = (int32_t)std::min<int64_t>(kPfCutSlots, L.pf_slots / 2);
     mla_prefill_kernel<<<(unsigned)L.pf_unit_cap, kPfWaves * 64, 0, s>>>(pa);
     if (int rc = check_hip(hipGetLastError(), "mla_prefill_kernel launch")) return rc;
   }

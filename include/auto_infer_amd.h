@@ -140,7 +140,8 @@ int aia_attn_plan(const int32_t* cu_seqlens_q, const int32_t* seqlens_kv,
  * from the rows themselves, saving the separate write launch.
  * Rows whose keys were split over several work-groups are merged by
  * log-sum-exp in a second kernel, from fp16 partials y = O / c scaled per
- * row (c = the row's largest |O|) with fp32 (max + log2 c, sum / c).
+ * row (c = the row's largest |O|) with fp32 (max + log2 c, sum / c).  Prompt
+ * rows that are cut only to even out the work-groups have fp32 partials.
  * flags: AIA_ATTN_KV_NZ -- the caches are in the NZ layout of the
  * reference's graph mode (gqa.py:163,202-226; see aia_kv_write_nz); the
  * fused KV write then writes that layout too.  Results are the same as with

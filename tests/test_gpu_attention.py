@@ -587,3 +587,65 @@ def test_ragged_prompts_dealt_largest_first(hq, hkv, d, lqs):
         span = max(8, hkv)
         assert all(min(size[i:i + span]) + bucket >= max(size[i + span:], default=0)
                    for i in range(0, jobs, span))
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs,lqs,jobs_above,plain", [
+    (14, 2, 64, 16, [1657, 40, 900, 333, 150, 700, 520], 448, 26),   # whole items without it
+    (24, 3, 128, 16, [1600, 300, 300, 200], 448, 25),     # 512 / Hkv not whole
+    (24, 3, 128, 16, [1500, 200, 333, 120, 90], 448, 22),  # items cut for the fill too
+    (32, 8, 128, 128, [900, 800, 64], 448, 15),
+    (28, 4, 128, 128, [1500, 300, 200], 448, 24),         # the grid that split-K ranges share
+    (14, 2, 64, 32, [1657, 40, 500, 333, 1, 2], 448, 18),   # split-K rows in a launch of their own
+])
+def test_balance_cuts_keep_fp32_partials(hq, hkv, d, bs, lqs, jobs_above, plain):
+    """Ragged prompts whose items fill the chip uncut, or nearly, are cut for
+    balance: the longest unit gets shorter (`plain`: without the cut), within
+    two work-groups per CU.  Their sums stay fp32 on the way: half of V's dims
+    are 2^-26 of the others, below what an fp16 value scaled by its row's
+    largest can hold, and still come out as exact as bf16 probabilities and
+    outputs allow (2^-9 each, so 2^-6 with room for rows of few keys).  Items
+    that are cut to fill the chip have fp16 partials as before.  Only cut
+    items' units have partial slots, so they come first in the list."""
+    s = workloads.make_gqa_step(lqs=lqs, lks=[lq + 5 * i for i, lq in enumerate(lqs)],
+                                num_q_heads=hq, num_kv_heads=hkv, head_dim=d, block_size=bs,
+                                seed=len(lqs))
+    s.v_cache[..., d // 2:] *= 2.0 ** -26
+    plan = ops.AttentionPlan.from_lists(s.block_table.to(DEV), s.cu_seqlens_q, s.seqlens_kv,
+                                        hq, hkv, d, bs)
+    out = torch.full(s.q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention_gqa(s.q.to(DEV), s.k_cache.to(DEV), s.v_cache.to(DEV), plan, s.scale,
+                            out=out)
+    # tokens of items with fp32 sums throughout (requests below one item are
+    # split-K's, whose partials are fp16)
+    group, rows = hq // hkv, torch.zeros(sum(lqs), dtype=torch.bool)
+    for i, lq in enumerate(lqs):
+        t0 = sum(lqs[:i])
+        if lq * group >= 128:
+            rows[t0:t0 + lq] = True
+        for r in range(0, lq * group, 128):
+            last = min(lq * group, r + 128) - 1
+            if -(-(5 * i + last // group + 1) // 64) > plain:
+                rows[t0 + r // group:t0 + last // group + 1] = False
+    got, ref = out.float().cpu(), oracle(s)
+    assert (got - ref).abs().max().item() <= TOL
+    got, ref = got[rows], ref[rows]
+    for part in (slice(0, d // 2), slice(d // 2, d)):
+        err = (got[..., part] - ref[..., part]).norm(dim=-1) / ref[..., part].norm(dim=-1)
+        assert err.max().item() <= 2.0 ** -6, (part, err.max().item())
+    L = ops.workspace_layout(len(lqs), sum(lqs), hq, hkv, d)
+    ws = plan.workspace.cpu()
+    hdr = ws[:64].view(torch.int32).tolist()
+    units, jobs = hdr[6], hdr[6] * hkv
+    assert hdr[8] == 0 and hdr[9] == jobs
+    assert jobs_above < jobs <= 512
+    rec = ws[L["pf"]:L["pf"] + 32 * units].view(torch.int32).view(units, 8)
+    mrg = ws[L["pfm"]:L["pfm"] + 16 * hdr[7]].view(torch.int32).view(hdr[7], 4)
+    cut = sum(int(k) & 0xffff for k in mrg[:, 3])
+    assert sorted(u for m in mrg.tolist() for u in range(m[2], m[2] + (m[3] & 0xffff))) == list(range(cut))
+    # fp32 ones first: those of the items that the fill alone leaves whole
+    sizes = {m[2]: int(rec[m[2]:m[2] + (m[3] & 0xffff), 3].max()) for m in mrg.tolist()}
+    assert 0 < hdr[11] <= cut
+    assert all((nt <= plain) == (u < hdr[11]) for u, nt in sizes.items())
+    assert cut <= min(512 // hkv, -(-448 // hkv))
+    assert 2 * cut * hkv * 128 * d * 2 <= L["total"] - L["pf_o"]
+    assert 8 * int((rec[:, 3] - rec[:, 2]).max()) <= 7 * plain

@@ -2550,11 +2550,16 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
           if (j0 + j >= k) break;
           const float mn = fmaxf(mx, ml[j].x);
           const float sa = __builtin_amdgcn_exp2f(mx - mn), sb = __builtin_amdgcn_exp2f(ml[j].x - mn);
-          ls = ls * sa + ml[j].y * sb;
-          acc[0].x = acc[0].x * sa + x[j][0].x * sb; acc[0].y = acc[0].y * sa + x[j][0].y * sb;
-          acc[0].z = acc[0].z * sa + x[j][0].z * sb; acc[0].w = acc[0].w * sa + x[j][0].w * sb;
-          acc[1].x = acc[1].x * sa + x[j][1].x * sb; acc[1].y = acc[1].y * sa + x[j][1].y * sb;
-          acc[1].z = acc[1].z * sa + x[j][1].z * sb; acc[1].w = acc[1].w * sa + x[j][1].w * sb;
+          // (the one rounding written out, so that it does not depend on how the
+          // compiler contracts either form)
+          ls = __builtin_fmaf(ls, sa, ml[j].y * sb);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            acc[i].x = __builtin_fmaf(acc[i].x, sa, x[j][i].x * sb);
+            acc[i].y = __builtin_fmaf(acc[i].y, sa, x[j][i].y * sb);
+            acc[i].z = __builtin_fmaf(acc[i].z, sa, x[j][i].z * sb);
+            acc[i].w = __builtin_fmaf(acc[i].w, sa, x[j][i].w * sb);
+          }
           mx = mn;
         }
       }

@@ -129,6 +129,7 @@ constexpr int kPfKeys = AIA_PF_KEYS;         // keys per staged K/V tile (32 or 
 #endif
 constexpr int kPfTargetWgs = AIA_PF_TARGET;
 constexpr int kPfCutSlots = 512;     // most work-groups (units x kv heads) of a step with cut items
+static_assert(kPfTargetWgs <= kPlanThreads && kPfCutSlots <= kPlanThreads, "a thread per cut item and unit");
 constexpr int kPfRecBytes = 48;      // a dealt work-group's record: three int4
 static_assert(2 * kPfTargetWgs >= kPfCutSlots && (2 * kPfTargetWgs - kPfCutSlots) * kPfRows * 8 >=
               kPfCutSlots * kPfRecBytes, "partials and records of a step with cut items");
@@ -403,6 +404,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   __shared__ int wave_sums[kPlanThreads / 64];
   __shared__ int2 wave_sums2[kPlanThreads / 64];
   __shared__ int pf_hist[64];
+  __shared__ int pf_longest;
+  __shared__ int4 pf_item[kPlanThreads];   // item f: {request, first row, tiles, units | first unit << 16}
+  __shared__ int pf_of[kPlanThreads];      // a unit's item
   const int tid = threadIdx.x;
   const int per_req = g.nkvg * g.nhb;
   // request metadata in LDS when it fits, else in the workspace / inputs
@@ -416,6 +420,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // get no segments and list their prefill items instead (last rows first:
   // under the causal mask they see the most keys)
   int carry = 0, pcarry = 0;
+  int most = 0;      // tiles of the longest item: a request's last one sees all its keys
+  if (tid < 64) pf_hist[tid] = 0;
+  if (tid == 0) pf_longest = 0;
   for (int base = 0; base < batch; base += kPlanThreads) {
     const int b = base + tid;
     int cnt = 0, pcnt = 0;
@@ -426,9 +433,10 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         if (b == batch - 1) cuv[batch] = c1;
       }
       const int lq = c1 - c0;
-      if (g.pf && (int64_t)lq * g.group >= kPfRows)
+      if (g.pf && (int64_t)lq * g.group >= kPfRows) {
         pcnt = (lq * g.group + kPfRows - 1) / kPfRows;
-      else
+        most = max(most, (max(lk, 0) + kPfKeys - 1) / kPfKeys);
+      } else
         cnt = lq > 0 ? ((lq + g.qs - 1) / g.qs) * per_req : 0;
     }
     int2 tot2;
@@ -451,8 +459,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // the causal mask they see the most keys).  When items x kv heads leave
   // the chip underfilled, an item's tiles are cut into k balanced chunks of
   // about `chunk` tiles; its k units write partials and get a merge record.
-  // Every loop below runs over the flat item list (request-major, each
-  // request's items last rows first), one item per thread.
+  // The loops below run over the flat item list (request-major, each
+  // request's items last rows first), one item per thread, then over the
+  // units.
   int units = 0, pmerges = 0, dealt = 0;
   int nwide = 0;            // units with fp32 partials
   // Fill target.  Absorbed-MLA units (158 KB of LDS) run one per CU: few
@@ -462,7 +471,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   const int pf_target = dv != 512 || g.ncu <= 0 || g.ncu >= kPfTargetWgs ? kPfTargetWgs
                         : (int64_t)pcarry * g.hkv <= g.ncu / 2 ? g.ncu : kPfTargetWgs;
   if (pcarry > 0) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
+    if ((tid & 63) == 0) atomicMax(&pf_longest, most);
     __syncthreads();   // item offsets
+    const int longest = pf_longest;
     const int* cu_p = req_lds ? cuv : cu_q;
     const int* kv_p = req_lds ? kvv : kvlen;
     // item f: its request, first row and key tiles
@@ -480,25 +493,37 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       const int kend = max(0, min(lk, lk - lq + last / g.group + 1));
       return (kend + kPfKeys - 1) / kPfKeys;
     };
+    // one item per thread: its request, row and tiles stay in registers
+    // through the searches below
+    const bool own = pcarry <= kPlanThreads;
+    int my_b = 0, my_r0 = 0, my_tiles = 0;
+    if (own && tid < pcarry) my_tiles = item_at(tid, my_b, my_r0);
+    auto item_tiles = [&](int f) {
+      if (own) return my_tiles;
+      int b, r0;
+      return item_at(f, b, r0);
+    };
     int chunk = 0x7fffffff, wtot = 0;
     int fill = 0;             // wide: the chunk that fills the chip
     bool wide = false;        // items of up to `fill` tiles are cut too
     // the least chunk above `lo` and up to `hi` whose units number at most
     // ucap, those of cut items at most ccap
+    auto fits = [&](int c, int ucap, int ccap) {
+      int nu = 0, nc = 0;
+      for (int f = tid; f < pcarry; f += kPlanThreads) {
+        const int nt = item_tiles(f);
+        const int k = nt > c ? (nt + c - 1) / c : 1;
+        nu += k;
+        nc += k > 1 ? k : 0;
+      }
+      int2 tot2;
+      block_exclusive_scan2(make_int2(nu, nc), wave_sums2, &tot2);
+      return tot2.x <= ucap && tot2.y <= ccap;
+    };
     auto least_chunk = [&](int lo, int hi, int ucap, int ccap) {
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        int nu = 0, nc = 0;
-        for (int f = tid; f < pcarry; f += kPlanThreads) {
-          int b, r0;
-          const int nt = item_at(f, b, r0);
-          const int k = nt > mid ? (nt + mid - 1) / mid : 1;
-          nu += k;
-          nc += k > 1 ? k : 0;
-        }
-        int2 tot2;
-        block_exclusive_scan2(make_int2(nu, nc), wave_sums2, &tot2);
-        if (tot2.x <= ucap && tot2.y <= ccap) hi = mid; else lo = mid + 1;
+        if (fits(mid, ucap, ccap)) hi = mid; else lo = mid + 1;
       }
       return hi;
     };
@@ -507,22 +532,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     const int pair_slots = min(2 * g.ncu, kPfCutSlots);
     const bool alone = carry == 0 || (dv != 512 && !mixed_grid(g, dv));
     const bool even = dv != 512 && alone && (int64_t)pcarry * g.hkv < pair_slots;
-    int mine = 0, most = 0;
-    for (int f = tid; f < pcarry; f += kPlanThreads) {
-      int b, r0;
-      const int nt = item_at(f, b, r0);
-      mine += nt;
-      most = max(most, nt);
+    if (even || (int64_t)pcarry * g.hkv < pf_target) {
+      int mine = 0;
+      for (int f = tid; f < pcarry; f += kPlanThreads) mine += item_tiles(f);
+      block_exclusive_scan(mine, wave_sums, &wtot);
     }
-    block_exclusive_scan(mine, wave_sums, &wtot);
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
-    if (tid == 0) pf_hist[0] = 0;
-    __syncthreads();
-    if ((tid & 63) == 0) atomicMax(&pf_hist[0], most);
-    __syncthreads();
-    const int longest = pf_hist[0];                  // tiles of the longest item
-    __syncthreads();
     if ((int64_t)pcarry * g.hkv < pf_target) {
       // sum_i ceil(nt_i / c) <= W / c + P, so c = W Hkv / (target - P Hkv)
       // keeps units x kv heads within the target: one round of work-groups
@@ -549,63 +563,58 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     // are cut for the fill too, then the whole ones, so that only cut items'
     // units have partial slots.
     if (even) {
-      const int ucap = pair_slots / g.hkv, top = min(longest, chunk);
-      const int c2 = least_chunk(min(top, max(kPfMinChunk, (wtot + ucap - 1) / ucap)), top, ucap,
-                                 min(ucap, pf_mrg_cap));
-      if (8 * c2 <= 7 * top) {
+      const int ucap = pair_slots / g.hkv, ccap = min(ucap, pf_mrg_cap);
+      const int top = (int)((int64_t)7 * min(longest, chunk) / 8);
+      const int lo = max(kPfMinChunk, (wtot + ucap - 1) / ucap);
+      if (lo <= top && fits(top, ucap, ccap)) {
         fill = chunk;
-        chunk = c2;
+        chunk = least_chunk(lo, top, ucap, ccap);
         wide = true;
       }
     }
-    int ucarry = 0, mcarry2 = 0;
-    for (int base = 0; base < pcarry; base += kPlanThreads) {
-      const int f = base + tid;
-      int b = 0, r0 = 0, nt = 0, k = 0;
-      if (f < pcarry) {
-        nt = item_at(f, b, r0);
-        k = nt > chunk ? (nt + chunk - 1) / chunk : 1;
-      }
+    // Units and merge records.  Items are cut only in steps of fewer items
+    // than threads (see kPfCutSlots); thread f then lists item f's units in
+    // LDS.  Larger steps have one unit per item.
+    if (own) {
+      const int nt = my_tiles, k = tid >= pcarry ? 0 : nt > chunk ? (nt + chunk - 1) / chunk : 1;
       const int kc = k > 1 ? k : 0, kw = wide && nt <= fill ? kc : 0;   // units of a cut item, fp32
       int2 tot2;
-      // (units of cut items and their records stay below 1024; wide steps have
-      // at most 512 units)
       const int2 ex2 = block_exclusive_scan2(make_int2(k | kw << 16, kc << 10 | (k > 1)), wave_sums2, &tot2);
-      const int mm = mcarry2 + (ex2.y & 1023);
-      int u = ucarry + ex2.x;
-      if (wide) {     // (fewer items than threads: one round lists them all)
-        const int w_before = ex2.x >> 16, c_before = ex2.y >> 10;
-        nwide = tot2.x >> 16;
-        tot2.x &= 0xffff;
-        u = kw ? w_before : kc ? nwide + c_before - w_before : (tot2.y >> 10) + (ex2.x & 0xffff) - c_before;
-      }
-      if (f < pcarry && u + k <= pf_unit_cap && mm + (k > 1) <= pf_mrg_cap) {
+      const int all_before = ex2.x & 0xffff, w_before = ex2.x >> 16, c_before = ex2.y >> 10;
+      const int mm = ex2.y & 1023;
+      units = tot2.x & 0xffff;
+      nwide = tot2.x >> 16;
+      pmerges = tot2.y & 1023;
+      const int u = !wide ? all_before : kw ? w_before : kc ? nwide + c_before - w_before
+                                                             : (tot2.y >> 10) + all_before - c_before;
+      if (units > kPlanThreads || units > pf_unit_cap || pmerges > pf_mrg_cap) {
+        units = 0; pmerges = 0; nwide = 0; overflow = 1;
+      } else if (tid < pcarry) {
+        pf_item[tid] = make_int4(my_b, my_r0, nt, k | u << 16);
+        for (int j = 0; j < k; ++j) pf_of[u + j] = tid;
         if (k > 1) {
           // {first query token, first row, first unit, units | item rows << 16}
-          const int c0 = req_lds ? cuv[b] : cu_q[b];
-          const int c1 = req_lds ? cuv[b + 1] : cu_q[b + 1];
-          const int rows = min(kPfRows, (c1 - c0) * g.group - r0);
-          pf_mrg[mm] = make_int4(c0, r0, u, k | (rows << 16));
-        }
-        // unit record: {request, first row, first tile, end tile}, then
-        // {first query token, query tokens, keys, block id of the first
-        // tile}, so a work-group starts its Q and first-tile loads as soon
-        // as its record arrives (the id serves block sizes that are a
-        // multiple of the tile)
-        const int c0 = cu_p[b], lqb = cu_p[b + 1] - c0, lkb = kv_p[b];
-        const int32_t* btr = block_table + (int64_t)b * bt_stride;
-        for (int j = 0; j < k; ++j) {
-          const int tj = (int)((int64_t)j * nt / k);
-          pf_units[2 * (u + j)] = make_int4(b, r0, tj, (int)((int64_t)(j + 1) * nt / k));
-          pf_units[2 * (u + j) + 1] = make_int4(c0, lqb, lkb, btr[(tj * kPfKeys) / block_size]);
+          const int c0 = cu_p[my_b], rows = min(kPfRows, (cu_p[my_b + 1] - c0) * g.group - my_r0);
+          pf_mrg[mm] = make_int4(c0, my_r0, u, k | (rows << 16));
         }
       }
-      ucarry += tot2.x;
-      mcarry2 += tot2.y & 1023;
+      __syncthreads();   // the units' items
+    } else {
+      units = pcarry;
+      if (units > pf_unit_cap) { units = 0; overflow = 1; }
     }
-    units = ucarry;
-    pmerges = mcarry2;
-    if (units > pf_unit_cap || pmerges > pf_mrg_cap) { units = 0; pmerges = 0; overflow = 1; }
+    // unit u's {request, first row, first tile, end tile}
+    auto unit_at = [&](int u) {
+      int b, r0;
+      if (!own) {
+        const int nt = item_at(u, b, r0);
+        return make_int4(b, r0, 0, nt);
+      }
+      const int4 i = pf_item[pf_of[u]];
+      const int k = i.w & 0xffff, j = u - (i.w >> 16);
+      if (k == 1) return make_int4(i.x, i.y, 0, i.z);
+      return make_int4(i.x, i.y, (int)((int64_t)j * i.z / k), (int)((int64_t)(j + 1) * i.z / k));
+    };
 
     // 1c) Work-group b's record at pf_wg[3 b]: its unit record (two int4),
     // then {unit, kv head}, so a work-group loads it beside the header
@@ -632,65 +641,63 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     const int jobs = units * g.hkv;
     const bool lpt = (dv == 512 && AIA_MLA_LPT) || jobs > 2 * g.ncu;
     const bool pair_deal = !lpt && alone && jobs > g.ncu && jobs <= 2 * g.ncu;
-    if (!pair_deal && !lpt) {
-      __syncthreads();   // publishes pf_units to the whole group
-      const int q = jobs / kXcdsPlan, r = jobs - q * kXcdsPlan;
-      for (int id = tid; id < jobs; id += kPlanThreads) {
-        const int x = id % kXcdsPlan, i = id / kXcdsPlan;
-        const int pair = x * q + min(x, r) + i;          // the run of XCD id % 8
-        const int kvh = pair / units, u = pair - kvh * units;
+    // units by size: 64 buckets of sizes up to the longest item's, bucket 0
+    // the largest, counting (unit, kv head) pairs or, largest first, units
+    auto bucket = [&](int nt) { return 63 - (int)min(64u * (unsigned)nt / (unsigned)(longest + 1), 63u); };
+    if (pair_deal || lpt) {
+      for (int u = tid; u < units; u += kPlanThreads) {
+        const int4 e = unit_at(u);
+        atomicAdd(&pf_hist[bucket(e.w - e.z)], lpt ? 1 : g.hkv);
+      }
+      __syncthreads();
+      if (tid < 64) {
+        const int c = pf_hist[tid];
+        pf_hist[tid] = wave_incl_scan(c) - c;
+      }
+      __syncthreads();
+    }
+    const int n2 = jobs - g.ncu, lone = g.ncu - n2;
+    const int per = kXcdsPlan / g.hkv, hpx = g.hkv / kXcdsPlan;
+    const int q = jobs / kXcdsPlan, longer = jobs - q * kXcdsPlan;   // runs of q + 1 pairs, then q
+    for (int p = tid; p < (lpt ? units : jobs); p += kPlanThreads) {
+      const int first = lpt ? 0 : p / units, u = p - first * units;
+      // unit record: {request, first row, first tile, end tile}, then
+      // {first query token, query tokens, keys, block id of the first
+      // tile}, so a work-group starts its Q and first-tile loads as soon
+      // as its record arrives (the id serves block sizes that are a
+      // multiple of the tile)
+      const int4 e = unit_at(u);
+      const int c0 = cu_p[e.x];
+      const int4 e2 = make_int4(c0, cu_p[e.x + 1] - c0, kv_p[e.x],
+                                block_table[(int64_t)e.x * bt_stride + (e.z * kPfKeys) / block_size]);
+      if (first == 0) {
+        pf_units[2 * u] = e;
+        pf_units[2 * u + 1] = e2;
+      }
+      const int rank = pair_deal || lpt ? atomicAdd(&pf_hist[bucket(e.w - e.z)], 1) : 0;
+      for (int kvh = first; kvh < (lpt ? g.hkv : first + 1); ++kvh) {
+        int id;
+        if (lpt) {
+          id = rank * g.hkv + kvh;
+          if (hpx * kXcdsPlan == g.hkv) {
+            id = kXcdsPlan * (rank * hpx + kvh % hpx) + kvh / hpx;
+          } else if (per * g.hkv == kXcdsPlan && rank < units - units % per) {
+            id = kXcdsPlan * (rank / per) + kvh * per + rank % per;
+          }
+        } else if (pair_deal) {
+          const int i = rank - lone;
+          id = rank < lone ? n2 + rank : i < n2 ? i : g.ncu + (jobs - 1 - rank);
+        } else {
+          const int x = p < longer * (q + 1) ? p / (q + 1) : longer + (p - longer * (q + 1)) / q;
+          id = kXcdsPlan * (p - x * q - min(x, longer)) + x;
+        }
         int4* rec = pf_wg + 3 * (int64_t)id;
-        rec[0] = pf_units[2 * u];
-        rec[1] = pf_units[2 * u + 1];
+        rec[0] = e;
+        rec[1] = e2;
         rec[2] = make_int4(u, kvh, 0, 0);
       }
-      dealt = jobs;
     }
-    if (pair_deal || lpt) {
-      if (tid < 64) pf_hist[tid] = 0;
-      __syncthreads();   // also publishes pf_units to the whole group
-      // 64 buckets of sizes up to the longest item's, bucket 0 the largest
-      auto bucket = [&](int nt) { return 63 - (int)min(64u * (unsigned)nt / (unsigned)(longest + 1), 63u); };
-      const int heads = lpt ? 1 : g.hkv, listed = units * heads;   // pairs sorted
-      for (int p = tid; p < listed; p += kPlanThreads) {
-        const int4 e = pf_units[2 * (p % units)];
-        atomicAdd(&pf_hist[bucket(e.w - e.z)], 1);
-      }
-      __syncthreads();
-      if (tid == 0) {
-        int acc = 0;
-        for (int k = 0; k < 64; ++k) { const int c = pf_hist[k]; pf_hist[k] = acc; acc += c; }
-      }
-      __syncthreads();
-      const int n2 = jobs - g.ncu, lone = g.ncu - n2;
-      const int per = kXcdsPlan / g.hkv, hpx = g.hkv / kXcdsPlan;
-      for (int p = tid; p < listed; p += kPlanThreads) {
-        const int u = p % units;
-        const int4 e = pf_units[2 * u], e2 = pf_units[2 * u + 1];
-        const int r = atomicAdd(&pf_hist[bucket(e.w - e.z)], 1);
-        auto put = [&](int id, int kvh) {
-          int4* rec = pf_wg + 3 * (int64_t)id;
-          rec[0] = e;
-          rec[1] = e2;
-          rec[2] = make_int4(u, kvh, 0, 0);
-        };
-        if (!lpt) {
-          const int i = r - lone;
-          put(r < lone ? n2 + r : i < n2 ? i : g.ncu + (jobs - 1 - r), p / units);
-          continue;
-        }
-        for (int kvh = 0; kvh < g.hkv; ++kvh) {
-          int id = r * g.hkv + kvh;
-          if (hpx * kXcdsPlan == g.hkv) {
-            id = kXcdsPlan * (r * hpx + kvh % hpx) + kvh / hpx;
-          } else if (per * g.hkv == kXcdsPlan && r < units - units % per) {
-            id = kXcdsPlan * (r / per) + kvh * per + r % per;
-          }
-          put(id, kvh);
-        }
-      }
-      dealt = jobs;
-    }
+    dealt = jobs;
   }
   __syncthreads();
   const int nseg = req_off[batch];

@@ -404,7 +404,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   __shared__ int wave_sums[kPlanThreads / 64];
   __shared__ int2 wave_sums2[kPlanThreads / 64];
   __shared__ int pf_hist[64];
-  __shared__ int pf_longest;
   __shared__ int4 pf_item[kPlanThreads];   // item f: {request, first row, tiles, units | first unit << 16}
   __shared__ int pf_of[kPlanThreads];      // a unit's item
   const int tid = threadIdx.x;
@@ -421,8 +420,6 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // under the causal mask they see the most keys)
   int carry = 0, pcarry = 0;
   int most = 0;      // tiles of the longest item: a request's last one sees all its keys
-  if (tid < 64) pf_hist[tid] = 0;
-  if (tid == 0) pf_longest = 0;
   for (int base = 0; base < batch; base += kPlanThreads) {
     const int b = base + tid;
     int cnt = 0, pcnt = 0;
@@ -473,9 +470,13 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   if (pcarry > 0) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
-    if ((tid & 63) == 0) atomicMax(&pf_longest, most);
+    if ((tid & 63) == 0) wave_sums[tid >> 6] = most;
+    if (tid < 64) pf_hist[tid] = 0;
     __syncthreads();   // item offsets
-    const int longest = pf_longest;
+    int longest = 0;
+#pragma unroll
+    for (int w = 0; w < kPlanThreads / 64; ++w) longest = max(longest, wave_sums[w]);
+    __syncthreads();   // (the scans below write the waves' places)
     const int* cu_p = req_lds ? cuv : cu_q;
     const int* kv_p = req_lds ? kvv : kvlen;
     // item f: its request, first row and key tiles
@@ -493,29 +494,20 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
       const int kend = max(0, min(lk, lk - lq + last / g.group + 1));
       return (kend + kPfKeys - 1) / kPfKeys;
     };
-    // one item per thread: its request, row and tiles stay in registers
-    // through the searches below
+    // Up to one item per thread: its request, row and tiles stay in registers
+    // through the searches below (items are cut only in such steps, see
+    // kPfCutSlots)
     const bool own = pcarry <= kPlanThreads;
     int my_b = 0, my_r0 = 0, my_tiles = 0;
     if (own && tid < pcarry) my_tiles = item_at(tid, my_b, my_r0);
-    auto item_tiles = [&](int f) {
-      if (own) return my_tiles;
-      int b, r0;
-      return item_at(f, b, r0);
-    };
     int chunk = 0x7fffffff, wtot = 0;
     int fill = 0;             // wide: the chunk that fills the chip
     bool wide = false;        // items of up to `fill` tiles are cut too
     // the least chunk above `lo` and up to `hi` whose units number at most
     // ucap, those of cut items at most ccap
     auto fits = [&](int c, int ucap, int ccap) {
-      int nu = 0, nc = 0;
-      for (int f = tid; f < pcarry; f += kPlanThreads) {
-        const int nt = item_tiles(f);
-        const int k = nt > c ? (nt + c - 1) / c : 1;
-        nu += k;
-        nc += k > 1 ? k : 0;
-      }
+      const int nu = tid >= pcarry ? 0 : my_tiles > c ? (my_tiles + c - 1) / c : 1;
+      const int nc = nu > 1 ? nu : 0;
       int2 tot2;
       block_exclusive_scan2(make_int2(nu, nc), wave_sums2, &tot2);
       return tot2.x <= ucap && tot2.y <= ccap;
@@ -532,11 +524,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     const int pair_slots = min(2 * g.ncu, kPfCutSlots);
     const bool alone = carry == 0 || (dv != 512 && !mixed_grid(g, dv));
     const bool even = dv != 512 && alone && (int64_t)pcarry * g.hkv < pair_slots;
-    if (even || (int64_t)pcarry * g.hkv < pf_target) {
-      int mine = 0;
-      for (int f = tid; f < pcarry; f += kPlanThreads) mine += item_tiles(f);
-      block_exclusive_scan(mine, wave_sums, &wtot);
-    }
+    if (even || (int64_t)pcarry * g.hkv < pf_target) block_exclusive_scan(my_tiles, wave_sums, &wtot);
     if ((int64_t)pcarry * g.hkv < pf_target) {
       // sum_i ceil(nt_i / c) <= W / c + P, so c = W Hkv / (target - P Hkv)
       // keeps units x kv heads within the target: one round of work-groups
@@ -572,9 +560,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         wide = true;
       }
     }
-    // Units and merge records.  Items are cut only in steps of fewer items
-    // than threads (see kPfCutSlots); thread f then lists item f's units in
-    // LDS.  Larger steps have one unit per item.
+    // Units and merge records: thread f lists item f's units in LDS.  Larger
+    // steps have one unit per item.
     if (own) {
       const int nt = my_tiles, k = tid >= pcarry ? 0 : nt > chunk ? (nt + chunk - 1) / chunk : 1;
       const int kc = k > 1 ? k : 0, kw = wide && nt <= fill ? kc : 0;   // units of a cut item, fp32

@@ -2274,10 +2274,11 @@ __global__ __launch_bounds__(64 * kMergeGroups) void merge_kernel(MergeArgs a) {
                                       : reinterpret_cast<const int4*>(a.hdr)) + vz;
   const int4* pp0 = (a.pf_mrg && item0 < a.pf_items_cap ? a.pf_mrg + (int)blockIdx.x / per_rec
                                                           : reinterpret_cast<const int4*>(a.hdr)) + vz;
-  const int* hv = a.hdr + vz;
+  const int4* hv = reinterpret_cast<const int4*>(a.hdr) + vz;
   const int4 m0_v = mp[0], m1_v = mp[1];
   const int4 pr_v = pp0[0];
-  const int h0 = hv[0], h2 = hv[2], h5 = hv[5], h7 = hv[7], h8 = hv[8], h10 = hv[10], h11 = hv[11];
+  const int4 h0_3 = hv[0], h4_7 = hv[1], h8_11 = hv[2];
+  const int h0 = h0_3.x, h2 = h0_3.z, h5 = h4_7.y, h7 = h4_7.w, h8 = h8_11.x, h10 = h8_11.z, h11 = h8_11.w;
   auto fold_into = [](float& mx, float& ls, float4 (&acc)[kMergeDims / 4], float2 ml,
                       const float4 (&x)[kMergeDims / 4]) {
     const float mn = fmaxf(mx, ml.x);
@@ -3345,8 +3346,9 @@ void mla_prefill_kernel(PrefillArgs a) {
   }
 }
 
+// max_keys: the context length that the block tables have room for.
 int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32_t dv, int32_t batch,
-                 int32_t tokens, int32_t waves,
+                 int32_t tokens, int32_t waves, int64_t max_keys,
                  const uint16_t* part_o,
                  const float2* part_ml, const int32_t* seg, uint16_t* out, int64_t o_ts,
                  int64_t o_hs, hipStream_t s) {
@@ -3358,21 +3360,38 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   mg.mrg = reinterpret_cast<const int32_t*>(ws + L.mrg); mg.mrg_cap = L.mrg_cap;
   const bool pf = L.pf_mrg_cap > 0;
   mg.pf_mrg = pf ? reinterpret_cast<const int4*>(ws + L.pfm) : nullptr;
-  // wide: 64-element slices (MLA, or 8+ rows per segment) and about 8 or
-  // more ranges per segment, i.e. a dozen partials per item
+  // elements of a segment's row span, with at least one query token per request
+  const int64_t nq_max = std::min<int64_t>(g.qs, (int64_t)tokens - batch + 1);
+  const int64_t rows_max = std::min<int64_t>(
+      (int64_t)kRows * g.rb, nq_max <= g.qb ? nq_max * g.hb : (int64_t)kRows * ((nq_max + g.qb - 1) / g.qb));
+  const int64_t span_max = nq_max >= 1 ? rows_max * (dv / kMergeDims) : kRows * g.rb * (dv / kMergeDims);
+  const int64_t blocks = std::max<int64_t>(batch, (tokens + g.qs - 1) / g.qs);
   // deep: few segments over many ranges each (a handful of long requests).
   // A record's 64 elements then go to eight work-groups, one row of head_dim
   // 128 each, whose lane groups fold 32 parts at a time instead of 4 or 8:
   // with whole slices a few work-groups walked hundreds of parts (one request
   // of 32K keys, 28/4 heads: 512 parts on 4 work-groups, 57 us per call; 21.7
   // with eighths.  16 latent heads, 32K keys: 54.9 -> 27.0).  At 64 ranges per
-  // segment eighths win everywhere (28/4 heads x 8 requests 37.2 -> 33.3, 64/8
-  // x 4 34.2 -> 32.0, 16/8 x 4 32.4 -> 31.4, 14/2 x 16 19.5 -> 17.5); at 32 they
-  // are between 34.6 -> 33.9 (28/4) and 48.7 -> 49.8 (16/8, whose whole slices
-  // have fixed slots), and at 16 52.1 -> 54.3: more work-groups than loads to
-  // spread.  (8 and 16 waves per work-group: slower.)
-  const int64_t blocks = std::max<int64_t>(batch, (tokens + g.qs - 1) / g.qs);
-  const bool deep = (int64_t)waves >= 64 * blocks * g.nkvg * g.nhb;
+  // segment eighths win for contexts of thousands of keys (28/4 heads x 8
+  // requests 37.2 -> 33.3, 64/8 x 4 34.2 -> 32.0, 16/8 x 4 32.4 -> 31.4, 14/2 x 16
+  // 19.5 -> 17.5); at 32 ranges they are between 34.6 -> 33.9 (28/4) and 48.7 ->
+  // 49.8 (16/8, whose whole slices have fixed slots), and at 16 52.1 -> 54.3:
+  // more work-groups than loads to spread.  (8 and 16 waves per work-group:
+  // slower.)
+  //   How many parts a segment has follows from the contexts, which only the
+  // device knows; the host knows what the block tables have room for.  Spans
+  // that fixed slots serve always have them up to kFixParts tiles, and one
+  // round trip less then beats eighths (16/8 heads, us per call, eighths
+  // against fixed slots: one request of 60 keys 9.9 / 9.3, of 500 10.4 / 9.6,
+  // of 1000, no fixed slots, 11.7 / 12.6; 4 requests of 250 11.3 / 10.6).  Other
+  // spans have little to fold up to 8 tiles (28/4 heads, eighths against whole
+  // slices: 60 keys 9.1 / 8.3, 100 9.1 / 8.6, 250 9.3 / 9.6, 500 9.5 / 11.0).  Short
+  // contexts in wide tables, as a gear has them, pay that difference.
+  const bool narrow = small_geometry(g, dv, batch, L.seg_cap) && span_max <= 16;
+  const bool deep = (int64_t)waves >= 64 * blocks * g.nkvg * g.nhb &&
+                    max_keys > kTile * (narrow ? kFixParts : 8);
+  // wide: 64-element slices (MLA, or 8+ rows per segment) and about 8 or
+  // more ranges per segment, i.e. a dozen partials per item
   const bool wide = AIA_MERGE_WIDE && !deep && L.pf_mrg_cap == 0 &&
                     (dv == kMlaV || (int64_t)g.hb * ((tokens + batch - 1) / batch) >= 8) &&
                     (int64_t)waves >= 8LL * batch * g.nkvg * g.nhb;
@@ -3396,14 +3415,9 @@ int launch_merge(char* ws, const Layout& L, const Geometry& g, int32_t nw, int32
   // loads per thread 40.6 -> 42 us, config 1 then 21.9 -> 22.75.)
   mg.fixed_slots = 0;
   mg.part_cap = L.part_cap;
-  if (!deep && small_geometry(g, dv, batch, L.seg_cap) && L.part_cap >= kFixParts * L.seg_cap) {
-    const int64_t nq_max = std::min<int64_t>(g.qs, (int64_t)tokens - batch + 1);
-    const int64_t rows_max = std::min<int64_t>(
-        (int64_t)kRows * g.rb, nq_max <= g.qb ? nq_max * g.hb : (int64_t)kRows * ((nq_max + g.qb - 1) / g.qb));
-    if (nq_max >= 1 && rows_max * (dv / kMergeDims) <= 16) {
-      mg.fixed_slots = 1;
-      mgrid = L.seg_cap * nw;
-    }
+  if (!deep && narrow && L.part_cap >= kFixParts * L.seg_cap) {
+    mg.fixed_slots = 1;
+    mgrid = L.seg_cap * nw;
   }
   if (mg.fixed_slots && !wide) {
     // kFixWaves waves of kFixParts / (4 kFixWaves) slot loads per thread (config 1,
@@ -3646,7 +3660,7 @@ extern "C" int aia_paged_attention_gqa(
   if (int rc = (flags & AIA_ATTN_KV_NZ) ? launch_gqa<true>(a, pa, L, g, head_dim, waves, one_block, s)
                                         : launch_gqa<false>(a, pa, L, g, head_dim, waves, one_block, s))
     return rc;
-  return launch_merge(ws, L, g, g.nw, head_dim, batch, num_tokens, waves, a.part_o, a.part_ml, a.seg, a.out, a.o_ts, a.o_hs,
+  return launch_merge(ws, L, g, g.nw, head_dim, batch, num_tokens, waves, (int64_t)block_table_stride * block_size, a.part_o, a.part_ml, a.seg, a.out, a.o_ts, a.o_hs,
                       s);
 }
 
@@ -3723,6 +3737,6 @@ extern "C" int aia_paged_attention_mla(
     mla_prefill_kernel<<<(unsigned)L.pf_unit_cap, kPfWaves * 64, 0, s>>>(pa);
     if (int rc = check_hip(hipGetLastError(), "mla_prefill_kernel launch")) return rc;
   }
-  return launch_merge(ws, L, g, 1, kMlaV, batch, num_tokens, waves, a.part_o, a.part_ml, a.seg, a.out, a.o_ts, a.o_hs,
+  return launch_merge(ws, L, g, 1, kMlaV, batch, num_tokens, waves, (int64_t)block_table_stride * block_size, a.part_o, a.part_ml, a.seg, a.out, a.o_ts, a.o_hs,
                       s);
 }

@@ -649,3 +649,26 @@ def test_balance_cuts_keep_fp32_partials(hq, hkv, d, bs, lqs, jobs_above, plain)
     assert cut <= min(512 // hkv, -(-448 // hkv))
     assert 2 * cut * hkv * 128 * d * 2 <= L["total"] - L["pf_o"]
     assert 8 * int((rec[:, 3] - rec[:, 2]).max()) <= 7 * plain
+
+
+@pytest.mark.parametrize("hq,hkv,d,lqs", [(16, 8, 128, [1, 1, 1]), (28, 4, 128, [1, 1]),
+                                          (14, 2, 64, [1, 1, 1, 1]), (32, 8, 128, [2, 1])])
+@pytest.mark.parametrize("columns", [0, 900])
+def test_short_contexts_with_narrow_and_wide_tables(hq, hkv, d, lqs, columns):
+    """A few requests of 30 to 400 keys: their plans have fixed partial slots
+    (header word 10) and more than one part per segment.  With tables that
+    hold little more than the contexts the merge takes whole slices or the
+    fixed slots, with wide ones eighths; the output is the same."""
+    lks = [400, 30, 257, 111][:len(lqs)]
+    s = workloads.make_gqa_step(lqs=lqs, lks=lks, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
+                                block_size=16, seed=hq)
+    bt = torch.zeros(len(lqs), max(columns, s.block_table.shape[1]), dtype=torch.int32)
+    bt[:, :s.block_table.shape[1]] = s.block_table
+    plan = ops.AttentionPlan.from_lists(bt.to(DEV), s.cu_seqlens_q, s.seqlens_kv, hq, hkv, d, 16)
+    out = torch.full(s.q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention_gqa(s.q.to(DEV), s.k_cache.to(DEV), s.v_cache.to(DEV), plan, s.scale,
+                            out=out)
+    hdr = plan.workspace[:64].cpu().view(torch.int32)
+    assert int(hdr[10]) == 1 and int(hdr[5]) > 0
+    err = (out.float().cpu() - oracle(s)).abs().max().item()
+    assert err <= TOL, err

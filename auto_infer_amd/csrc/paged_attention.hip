@@ -212,7 +212,9 @@ int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
 // reading a merge record, and issues those loads together with the
 // header's, one round trip instead of two.  hdr[10] = 1 marks such a plan.
 // Both planners decide it the same way, from the slot capacity the host
-// passes (fix_cap, 0 outside the geometry) and the ranges.
+// passes (fix_cap, 0 outside the geometry) and the ranges.  A step with an
+// empty request has no such plan: the host's bound on a segment's rows, by
+// which the merge's launch is chosen, takes one query token per request.
 constexpr int kFixParts = 32;
 #ifndef AIA_FIX_WAVES
 #define AIA_FIX_WAVES 2
@@ -419,6 +421,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // get no segments and list their prefill items instead (last rows first:
   // under the causal mask they see the most keys)
   int carry = 0, pcarry = 0;
+  bool empty = false;   // one of this thread's requests has no query token
   int most = 0;      // tiles of the longest item: a request's last one sees all its keys
   for (int base = 0; base < batch; base += kPlanThreads) {
     const int b = base + tid;
@@ -430,6 +433,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
         if (b == batch - 1) cuv[batch] = c1;
       }
       const int lq = c1 - c0;
+      empty = empty || lq <= 0;
       if (g.pf && (int64_t)lq * g.group >= kPfRows) {
         pcnt = (lq * g.group + kPfRows - 1) / kPfRows;
         most = max(most, (max(lk, 0) + kPfKeys - 1) / kPfKeys);
@@ -907,7 +911,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     }
     // fixed partial slots (see kFixParts), decided as the small planner does
     fixed = nseg <= kSmallPlanSegs && nseg * kFixParts <= fix_cap &&
-            !__syncthreads_or(np > kFixParts);
+            !__syncthreads_or(np > kFixParts || empty);
     int2 tot2;
     const int2 ex2 = block_exclusive_scan2(make_int2(np, mcnt), wave_sums2, &tot2);
     const int ex = ex2.x, tot = tot2.x, mex = ex2.y, mtot = tot2.y;
@@ -1100,9 +1104,11 @@ __global__ __launch_bounds__(kSmallPlanThreads) void plan_small_kernel(
   if (tid < 64) {
     // 1) segments per request (lane = request)
     int c0 = 0, c1 = 0, lk = 0, cnt = 0;
+    bool empty = false;
     if (lane < batch) {
       c0 = cu_q[lane]; c1 = cu_q[lane + 1]; lk = kvlen[lane];
       const int lq = c1 - c0;
+      empty = lq <= 0;
       cnt = lq > 0 ? ((lq + g.qs - 1) / g.qs) * per_req : 0;
     }
     const int inc = wave_incl_scan(cnt);
@@ -1177,7 +1183,7 @@ __global__ __launch_bounds__(kSmallPlanThreads) void plan_small_kernel(
     }
     const int pinc = wave_incl_scan(np), minc = wave_incl_scan(mcnt);
     // fixed partial slots (see kFixParts)
-    const bool fixed = nseg * kFixParts <= fix_cap && !__any(np > kFixParts);
+    const bool fixed = nseg * kFixParts <= fix_cap && !__any(np > kFixParts || empty);
     const int part_base = fixed ? kFixParts * s : pinc - np, mbase = minc - mcnt;
     const int nparts = fixed ? kFixParts * nseg : __builtin_amdgcn_readlane(pinc, 63);
     const int nmrg = __builtin_amdgcn_readlane(minc, 63);

@@ -672,3 +672,12 @@ def test_short_contexts_with_narrow_and_wide_tables(hq, hkv, d, lqs, columns):
     assert int(hdr[10]) == 1 and int(hdr[5]) > 0
     err = (out.float().cpu() - oracle(s)).abs().max().item()
     assert err <= TOL, err
+
+
+@pytest.mark.parametrize("lqs", [[2, 0], [1, 3, 0, 0, 1, 1], [2, 0, 1, 1, 1, 1, 0, 3, 1, 1]])
+def test_empty_requests_beside_longer_ones(lqs):
+    """The step's token count alone would say one token per request; an empty
+    request lets another have more, whose rows then need more than the 16
+    elements that a fixed-slot merge serves."""
+    check(workloads.make_gqa_step(lqs=lqs, lks=[(300 + 40 * i) if lq else 0 for i, lq in enumerate(lqs)],
+                                  num_q_heads=16, num_kv_heads=8, block_size=16, seed=len(lqs)))

@@ -2980,6 +2980,7 @@ void mla_prefill_kernel(PrefillArgs a) {
   __shared__ int btl[kMlaBtl];
   __shared__ float sl[kPfRows], sm[kPfRows], smax[kPfWaves][kPfRows];
   __shared__ int rerun_flag;
+  __shared__ int tlast[kMlaRT];          // last key that a 32-row tile sees
   const int wg = blockIdx.x;
   // this work-group's unit, as the GQA units take theirs (one kv head)
   const int4* rec = a.dealt + 3 * (int64_t)wg;
@@ -3058,6 +3059,8 @@ void mla_prefill_kernel(PrefillArgs a) {
   };
   const int lx0 = lane ^ (2 * (wid & 1));
 
+  if (tid < kMlaRT) tlast[tid] = min(ctx0 + (min(row_end, row0 + 32 * (tid + 1)) - 1) / G, lk - 1);
+
   // this wave's rows
   const int row = row0 + 32 * wid + n;
   const bool rv = row < row_end;
@@ -3102,10 +3105,16 @@ void mla_prefill_kernel(PrefillArgs a) {
   // those of the sub-tile after it; past the unit's last key they re-read it).
   // Without MASK every valid row sees all of sub-tile v's keys.
   int mine = 0;          // this lane's slot in the sub-tile to load next
+  // In masked steps and the last one PV of a row tile leaves out the keys past
+  // the tile's last visible one (P is zero there, but 0 x V is not where V is
+  // an infinity or NaN): row tiles go one after the other, the last first, and
+  // a wave clears its own dims of those keys in LDS before each.  (Kept in
+  // registers and masked per row tile instead, the fragments and masks made 7 KB
+  // more code, fetched once per unit, and the kernel 6 us slower.)
   auto step = [&](auto qk_tag, auto pv_tag, auto mask_tag, int v, int bk, int bv, int bn)
                   __attribute__((always_inline)) {
     constexpr bool QK = decltype(qk_tag)::value, PV = decltype(pv_tag)::value;
-    constexpr bool MASK = decltype(mask_tag)::value;
+    constexpr bool MASK = decltype(mask_tag)::value, EDGE = PV && (MASK || !QK);
     // opaque copies, so that the swizzled offsets are computed where they are
     // used (one xor each) instead of being kept, and spilled, across the loop
     int kx = kx0, rx = rx0, vx = vx0, lx = lx0;
@@ -3132,7 +3141,7 @@ void mla_prefill_kernel(PrefillArgs a) {
     u32x4_t pf[kMlaRT];
     bf16x8_t vf[3];
     auto pv_ahead = [&](int e) __attribute__((always_inline)) {     // PV's first operands, in 6 pieces
-      if (!PV) return;
+      if (!PV || EDGE) return;
       if (e < 4) pf[e] = read_p(0, e);
       else vf[e - 4] = read_v(e - 4);
     };
@@ -3193,6 +3202,29 @@ void mla_prefill_kernel(PrefillArgs a) {
         *reinterpret_cast<u32x4_t*>(d + 2 * kPfRows * 16) = u32x4_t{pk[4], pk[5], pk[6], pk[7]};
       }
     };
+    if (EDGE) {
+      int past = kMlaSub;                             // keys from here on are cleared
+#pragma unroll
+      for (int rt = kMlaRT - 1; rt >= 0; --rt) {
+        const int seen = max(__builtin_amdgcn_readfirstlane(tlast[rt]) - (v - 1) * kMlaSub + 1, 0);
+        char* own = const_cast<char*>(vt) + 256 * wid + 4 * lane;
+        for (int k = seen; k < past; ++k) *reinterpret_cast<uint32_t*>(own + 1024 * k) = 0;
+        past = min(past, seen);
+        pf[0] = read_p(0, rt);
+        pf[1] = read_p(1, rt);
+        vf[0] = read_v(0);
+        vf[1] = read_v(1);
+#pragma unroll
+        for (int f = 0; f < 8; ++f) {
+          if (f + 2 < 8) vf[(f + 2) % 3] = read_v(f + 2);
+          o[f & 3][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              vf[f % 3], __builtin_bit_cast(bf16x8_t, pf[f >> 2]), o[f & 3][rt], 0, 0, 0);
+          soft(8 * (kMlaRT - 1 - rt) + f);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
       if (PV) {

@@ -251,3 +251,26 @@ def test_mla_prefill_unit_reruns_with_exact_row_maxima():
     step.q_latent = (step.q_latent.float() * 40).to(torch.bfloat16)
     print("mla prefill units with scores spread past 2^64", flush=True)
     check(step)
+
+
+@pytest.mark.parametrize("heads,reach", [(1, 32), (3, 12), (16, 2), (64, 1)])
+@pytest.mark.parametrize("lqs,lks,token", [([200], [200], 138), ([257], [1300], 196), ([160], [9000], 159),
+                                           ([133, 140], [133, 175], 17)])
+def test_mla_prefill_units_keep_non_finite_latents_to_their_rows(heads, reach, lqs, lks, token):
+    """An infinity and a NaN in a later token's latent: the rows of a 32-row
+    tile that sees the key take it up (0 x infinity in masked places too), no
+    other row changes by a bit.  A tile spans `reach` tokens at most."""
+    step = workloads.make_mla_step(lqs=lqs, lks=lks, num_heads=heads, block_size=16, seed=heads)
+    s = step
+    plan = ops.AttentionPlan.from_lists(s.block_table.to(DEV), s.cu_seqlens_q, s.seqlens_kv, heads,
+                                        1, 512, 16)
+    pos = lks[0] - lqs[0] + token
+    clean = ops.paged_attention_mla(s.q_latent.to(DEV), s.cache.to(DEV), plan, s.scale).cpu()
+    bad = s.cache.clone()
+    row = bad[s.block_table[0, pos // 16], pos % 16].view(-1)
+    row[5], row[300] = float("inf"), float("nan")
+    out = ops.paged_attention_mla(s.q_latent.to(DEV), bad.to(DEV), plan, s.scale).cpu()
+    assert plan.workspace[:64].cpu().view(torch.int32)[6] > 0       # prefill units
+    same = (out.view(torch.int16) == clean.view(torch.int16)).flatten(1).all(1)
+    assert bool(same[:max(0, token - reach + 1)].all()) and bool(same[lqs[0]:].all())
+    assert not bool(out[token:lqs[0], :, [5, 300]].isfinite().any())

@@ -2959,6 +2959,10 @@ static_assert(kPfWaves == 4 && kPfKeys == 2 * kMlaSub && kPfRows == 32 * kPfWave
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
 // S += K Q^T in VGPRs (see above); the first of a chain starts from zero.
+// The hazard recogniser does not see these as MFMAs, so they are right only
+// while the register allocator places no copy of S between two links, none of
+// a K or Q fragment directly in front of one, and no read of S before
+// mla_s_ready.  tests/test_native_lib.py checks that on the built kernel.
 __device__ __forceinline__ void mla_s_first(float16_t& s, u32x4_t k, u32x4_t q) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "v"(q));
 }

@@ -2,6 +2,7 @@
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -150,3 +151,70 @@ def test_error_messages_are_per_thread():
     for t in ts:
         t.join()
     assert not errs, errs[:3]
+
+
+def _kernel_assembly(tmp_path, name):
+    """Instructions (mnemonic, operands) of one kernel of the built library."""
+    bins = "/opt/rocm/llvm/bin/"
+    for tool in ("llvm-objcopy", "clang-offload-bundler", "llvm-objdump"):
+        if not os.path.exists(bins + tool):
+            pytest.skip(f"no {tool}")
+    fat, out = str(tmp_path / "fat"), []
+    subprocess.run([bins + "llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", _native.LIB_PATH,
+                    str(tmp_path / "copy")], check=True)
+    # one bundle per source file, each aligned to a page behind its magic
+    data = open(fat, "rb").read()
+    starts = [m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)]
+    for i, a in enumerate(starts):
+        part, obj = str(tmp_path / f"part{i}"), str(tmp_path / f"obj{i}")
+        open(part, "wb").write(data[a:(starts + [len(data)])[i + 1]])
+        subprocess.run([bins + "clang-offload-bundler", "--type=o", "--unbundle", f"--input={part}",
+                        f"--output={obj}", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950"], check=True)
+        text = subprocess.run([bins + "llvm-objdump", "-d", "--mcpu=gfx950", obj], check=True,
+                              capture_output=True, text=True).stdout
+        inside = False
+        for line in text.splitlines():
+            if re.match(r"[0-9a-f]+ <", line):
+                inside = name in line
+            elif inside and line.strip():
+                op, _, rest = line.split("//")[0].strip().partition(" ")
+                out.append((op, [x.strip() for x in rest.split(",")]))
+    return out
+
+
+def _vgprs(operand):
+    m = re.fullmatch(r"[-|]*v(\d+)\|?", operand) or re.fullmatch(r"v\[(\d+):(\d+)\]", operand)
+    if not m:
+        return set()
+    return set(range(int(m[1]), int(m[m.lastindex]) + 1))
+
+
+def test_mla_score_mfmas_have_their_wait_states(tmp_path):
+    """The MLA prefill kernel issues QK^T as inline assembly, which the
+    compiler's hazard recogniser does not see as MFMAs.  In the built kernel:
+    no VALU instruction writes an operand of one within two wait states in
+    front of it; between the links of a chain nothing else reads or writes
+    the accumulator; and behind the last link its first other use is 11 wait
+    states away (an 8-pass MFMA's), an MFMA in between counting as its 8."""
+    code = _kernel_assembly(tmp_path, "mla_prefill_kernel")
+    assert code
+    states = [int(a[0], 0) + 1 if op == "s_nop" else 8 if op.startswith("v_mfma") else 1 for op, a in code]
+    links = [i for i, (op, a) in enumerate(code) if op.startswith("v_mfma") and _vgprs(a[0])]
+    chains = sum(code[i][1][3] == "0" for i in links)
+    assert chains >= 3 and len(links) == 36 * chains       # a first, a plain and a masked step
+    for n, i in enumerate(links):
+        acc, operands = _vgprs(code[i][1][0]), set().union(*map(_vgprs, code[i][1]))
+        waited, j = 0, i - 1
+        while waited < 2:
+            op, a = code[j]
+            if op.startswith("v_") and not op.startswith("v_mfma"):
+                written = _vgprs(a[0]) | (_vgprs(a[1]) if "swap" in op else set())
+                assert not written & operands, (code[j], code[i])
+            waited, j = waited + states[j], j - 1
+        last = n + 1 == len(links) or code[links[n + 1]][1][3] == "0"
+        stop = len(code) if last else links[n + 1]
+        waited, j = 0, i + 1
+        while j < stop and (not last or waited < 11):
+            op, a = code[j]
+            assert not set().union(*map(_vgprs, a)) & acc, (code[i], code[j], waited)
+            waited, j = waited + states[j], j + 1

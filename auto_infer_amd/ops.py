@@ -150,6 +150,13 @@ def mla_q_latent(q, w_uk_t, cos, sin, out=None):
     return out
 
 
+# Query rows (tokens x heads) up to which mla_v_up beats the library GEMM, for
+# programs that route by it: every count it takes, since long steps have a
+# kernel of their own (16 heads: 192 tokens 6.2 -> 4.9 us, 2450 tokens 55 ->
+# 12.9 against the library's 23.5).
+MLA_V_UP_MAX_ROWS = 2 ** 31 - 1
+
+
 def mla_v_up(o_latent, w_uv, out=None):
     """Absorbed-MLA value up-projection, one launch: ``einsum("tnl,nvl->tnv",
     o_latent[..., :512], W_UV)`` (auto_infer/layers/attention/mla.py:120-121)

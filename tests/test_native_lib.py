@@ -129,6 +129,13 @@ def test_argument_validation_of_the_fused_kernels_without_gpu():
     assert lib.aia_mla_q_latent(None, 0, 0, 0, 16, None, None, 0, None, 0, None, 0, 0, None) == 0
 
 
+def test_public_limits_of_the_ops():
+    """Names that programs route by stay: up to this many rows mla_v_up is the
+    faster way."""
+    from auto_infer_amd import ops
+    assert ops.MLA_V_UP_MAX_ROWS >= 4096
+
+
 def test_error_messages_are_per_thread():
     """aia_last_error() is thread local: two host threads failing with
     different arguments at the same time each read their own message."""

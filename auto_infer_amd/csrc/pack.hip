@@ -55,52 +55,73 @@ __global__ __launch_bounds__(256) void pack_updates_kernel(
 // dependent loads (descriptor, block id, store) whatever it moves, so its
 // length is what the kernel takes: one wave per row walked a 1991-column table
 // row, or a 1657-token prompt, 64 at a time (14-16 us; chunked, with a
-// chunk's loads issued before its stores, 3.6 us).
+// chunk's loads issued before its stores, 3.6 us).  Up to 64 values go one to
+// a lane: all four loads and stores of a chunk, masked, cost a decode row 0.3
+// to 0.5 us (16 rows inline: 2.9 us in one wave per row, 3.5 with whole chunks
+// only, 3.1 now; 256 rows of the staging copy 2.4, 2.8, 2.5).
 constexpr int kChunk = 256;
 constexpr int kMaxChunks = 64;     // a longer row's chunks go round
 
+// N x 64 tokens of a row from token j0 on.
+template <int N>
+__device__ __forceinline__ void pack_tokens(const PackArgs& a, const int32_t* prow, const int64_t* trow,
+                                            int base, int start, int n, int q_off, int j0, int lane) {
+  const int max_col = (int)a.block_stride - 1;
+  int blk[N], off[N];
+  int64_t tok[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int j = min(j0 + 64 * i + lane, n - 1);
+    const int bi = (start + j) / a.block_size;
+    off[i] = start + j - bi * a.block_size;
+    blk[i] = prow ? prow[min(bi, max_col)] : base + bi;
+    tok[i] = trow ? trow[min((int64_t)(start + j), a.token_stride - 1)] : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int j = j0 + 64 * i + lane;
+    if (j >= n) break;
+    const int64_t q = q_off + j;
+    a.positions[q] = start + j;
+    a.slot_mapping[q] = blk[i] * a.block_size + off[i];
+    a.token_ids[q] = tok[i];
+  }
+}
+
+// N x 64 columns of a block-table row from column c0 on.
+template <int N>
+__device__ __forceinline__ void pack_columns(const PackArgs& a, const int32_t* prow, int base,
+                                             int nblocks, int32_t* bt, int c0, int lane) {
+  const int last = min(nblocks, (int)a.block_stride) - 1;
+  int v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = base + c0 + 64 * i + lane;
+  if (prow && nblocks > 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = prow[min(c0 + 64 * i + lane, last)];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = c0 + 64 * i + lane;
+    if (c < a.bt_width) bt[c] = c < nblocks ? v[i] : 0;
+  }
+}
+
+// Chunks `chunk`, `chunk` + nchunks, ... of row r.
 __device__ __forceinline__ void pack_one_row(const PackArgs& a, int r, const int32_t* d, int lane,
                                              int chunk, int nchunks) {
-  constexpr int kPer = kChunk / 64;
   const int src = d[0], start = d[1], n = d[2], nblocks = d[3], base = d[4], q_off = d[5];
   const int zero_tokens = d[6], sample_slot = d[7];
   const int32_t* prow = src >= 0 ? a.block_pool + (int64_t)src * a.block_stride : nullptr;
-  const int64_t* trow = src >= 0 ? a.token_pool + (int64_t)src * a.token_stride : nullptr;
-  const int max_col = (int)a.block_stride - 1;
+  const int64_t* trow = src >= 0 && !zero_tokens ? a.token_pool + (int64_t)src * a.token_stride : nullptr;
   for (int j0 = chunk * kChunk; j0 < n; j0 += nchunks * kChunk) {
-    int blk[kPer], off[kPer];
-    int64_t tok[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int j = min(j0 + 64 * i + lane, n - 1);
-      const int bi = (start + j) / a.block_size;
-      off[i] = start + j - bi * a.block_size;
-      blk[i] = prow ? prow[min(bi, max_col)] : base + bi;
-      tok[i] = (zero_tokens || !trow) ? 0 : trow[min((int64_t)(start + j), a.token_stride - 1)];
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int j = j0 + 64 * i + lane;
-      if (j >= n) break;
-      const int64_t q = q_off + j;
-      a.positions[q] = start + j;
-      a.slot_mapping[q] = blk[i] * a.block_size + off[i];
-      a.token_ids[q] = tok[i];
-    }
+    if (n - j0 <= 64) pack_tokens<1>(a, prow, trow, base, start, n, q_off, j0, lane);
+    else pack_tokens<kChunk / 64>(a, prow, trow, base, start, n, q_off, j0, lane);
   }
   int32_t* bt = a.block_table + (int64_t)r * a.bt_width;
   for (int c0 = chunk * kChunk; c0 < a.bt_width; c0 += nchunks * kChunk) {
-    int v[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int c = c0 + 64 * i + lane;
-      v[i] = c < nblocks ? (prow ? prow[min(c, max_col)] : base + c) : 0;
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int c = c0 + 64 * i + lane;
-      if (c < a.bt_width) bt[c] = v[i];
-    }
+    if (a.bt_width - c0 <= 64) pack_columns<1>(a, prow, base, nblocks, bt, c0, lane);
+    else pack_columns<kChunk / 64>(a, prow, base, nblocks, bt, c0, lane);
   }
   if (lane == 0 && chunk == 0) {
     if (r == 0) a.cu_seqlens_q[0] = 0;
@@ -111,6 +132,7 @@ __device__ __forceinline__ void pack_one_row(const PackArgs& a, int r, const int
   }
 }
 
+// Rows of the staging copy, `nchunks` waves each.
 __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs a, int nchunks) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -127,7 +149,8 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs a, int nchunks)
 // kernel arguments (the launch copies them; no staging copy): the pool updates
 // first, then, after a work-group barrier, one wave per row chunk.  Every
 // work-group makes all the updates itself before it reads (the same values to
-// the same places, at most 192 of them), so none waits for another; a step of
+// the same places; 3 KB of arguments hold fewer than 256), so none waits for
+// another, and a step updates an entry at most once; a step of
 // up to 16 chunks is one work-group of 16 waves.  (64 rows of a latent gear in
 // one work-group took 11 us, four row passes of 16 waves; in four, 4.2.)
 template <int BYTES>
@@ -231,7 +254,9 @@ extern "C" int aia_pack_rows(const int64_t* token_update_index, const int64_t* t
   a.last_rows = last_rows; a.sample_rows = sample_rows;
   a.sample_count = sample_count; a.sample_cap = sample_cap;
   // The rows are on the device, so their token counts are not known here: the
-  // table's width gives the chunks, and at least four for a prompt's tokens.
+  // table's width gives the waves per row, and at least four for a prompt's
+  // tokens (4096 of one: 17.5 us in one wave, 5.2 in four).  Decode rows leave
+  // three of them idle: 0.1 us up to 500 rows, 0.4 at 1024.
   int nchunks = (block_table_width + kChunk - 1) / kChunk;
   nchunks = nchunks < 4 ? 4 : nchunks > kMaxChunks ? kMaxChunks : nchunks;
   const int64_t waves = (int64_t)num_rows * nchunks;

@@ -259,6 +259,8 @@ def test_build_of_each_inline_argument_size(batch):
     (1, [(0, 255), (3, 256), (0, 257), (900, 1)]),       # tables and prompts at a chunk's edges
     (16, [(0, 1657), (31000, 1), (5, 64)]),              # a long table beside a long prompt
     (1, [(0, 16500), (16700, 1)]),                       # more than 64 chunks: they go round
+    # waves that share the chunks of four rows, the last work-group of one row
+    (4, [(0, 64), (0, 65), (10, 1), (0, 256), (7, 257), (0, 1025), (63, 2), (1030, 1), (0, 1300)]),
 ])
 def test_build_rows_cut_into_chunks(bs, chunks, inline, monkeypatch):
     """Rows whose tokens and table columns span several waves' chunks; the

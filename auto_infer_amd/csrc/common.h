@@ -64,11 +64,12 @@ __device__ __forceinline__ float group4_sum(float x) {
 // (lds wave-uniform).  Issued as inline assembly on purpose: the compiler's
 // counter-wait pass tracks the builtin form as an outstanding LDS access and
 // then waits for the LDS counter to drain completely (lgkmcnt(0)) before
-// every LDS read, which exposes each read's full latency (48.2 against 49.3
-// µs per call, and it defeats the read-ahead order above: 47.6-47.9 against
-// 46.0).  Completion is explicit instead: every step waits vmcnt(0) before its
-// barrier.  Loads the compiler does not see can only make its own vmcnt waits
-// stricter, never too weak (the counter retires in order).
+// every LDS read, which exposes each read's full latency (the GQA prefill
+// units, us per call: 49.3 with the builtin against 48.2, and 47.6-47.9
+// against 46.0 with V read from LDS ahead of its use).  Completion is explicit
+// instead: a wave waits for its own loads (s_waitcnt vmcnt) before the barrier
+// that publishes their bytes.  Loads the compiler does not see can only make
+// its own vmcnt waits stricter, never too weak (the counter retires in order).
 // m0 (the LDS address of the load) is named as clobbered, which clang warns
 // about for a register it reserves: the warning is silenced here because the
 // clobber is what tells the compiler that m0 changed, and the compiler keeps

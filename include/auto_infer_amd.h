@@ -260,9 +260,10 @@ int aia_pack_rows(const int64_t* token_update_index, const int64_t* token_update
 
 /* aia_pack_rows for small steps, with no staging copy: the updates and row
  * descriptors come in `blob`, HOST memory that the call copies into the
- * kernel launch's arguments, and one work-group scatters the updates and
- * packs the rows.  blob layout (8-byte words): token_update_index [nt]
- * int64, token_update_value [nt] int64, block_update_index [nb] int64,
+ * kernel launch's arguments.  Every work-group scatters all the updates and
+ * then packs its share of the rows, so a pool entry is updated at most once
+ * in a call.  blob layout (8-byte words): token_update_index [nt] int64,
+ * token_update_value [nt] int64, block_update_index [nb] int64,
  * block_update_value [nb] int32 (padded to a whole word), rows [num_rows][8]
  * int32; at most AIA_PACK_INLINE_BYTES bytes (AIA_ERR_CAPACITY otherwise).
  * Other arguments and the outputs as in aia_pack_rows.  No reference

@@ -465,10 +465,13 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   // units.
   int units = 0, pmerges = 0, dealt = 0;
   int nwide = 0;            // units with fp32 partials
-  // Fill target.  Absorbed-MLA units (158 KB of LDS) run one per CU: few
-  // items are cut into one round of units (8 x 64 tokens at 4096 keys: 172
-  // us against 205 at 448), many into about 1.75 rounds so the causal
-  // items even out (1 x 2048 tokens: 218 against 280 at one round).
+  // Fill target.  Absorbed-MLA units (135 KB of LDS) run one per CU: few
+  // items are cut into one round of units, many into about 1.75 rounds so the
+  // causal items even out.  16 heads, us per call at one round / 448: 64
+  // items, 8 x 64 tokens at 4096 keys 92 / 118, 512 at 16K 263 / 292; 128
+  // items, 1024 at 8192 261 / 282; 256 items, 2048 tokens alone 128 / 123,
+  // four ragged prompts 104 / 102, but 4 x 512 at 4096, whose items are all
+  // long, 252 / 270; 368 items of five chunks 210 / 212.
   const int pf_target = dv != 512 || g.ncu <= 0 || g.ncu >= kPfTargetWgs ? kPfTargetWgs
                         : (int64_t)pcarry * g.hkv <= g.ncu / 2 ? g.ncu : kPfTargetWgs;
   if (pcarry > 0) {
@@ -2912,14 +2915,16 @@ void mla_attn_kernel(MlaArgs a) {
 //   LDS (8 KB per sub-tile).
 // The kernel is bound by what one wave per SIMD can issue.  A step's 68 MFMAs
 // take 2176 cycles and hide about six other instructions each; the step holds
-// some 480 and takes about 3400, 4600 cycles more go into a unit's first loads
-// and its output.  With 16 rows per wave in two passes of 64, QK^T, softmax and
+// some 480 and takes about 3400.  The rest of a unit is its first loads and its
+// output: 32 units of 2, 4, 8 and 16 steps each take 20.3, 23.6, 29.0 and 41.4
+// us, 1.5 a step and 17 with the launch of the kernel and its code's way from
+// memory.  With 16 rows per wave in two passes of 64, QK^T, softmax and
 // PV one after the other and V^T read by every wave (the form before), 2176
 // cycles of MFMA took 12000.  Here step v holds QK^T of sub-tile v and PV of
 // sub-tile v - 1, which do not depend on each other, and the softmax of v runs
 // between the MFMAs of PV.  16 heads, us per call with the merge, before -> now:
 // 2921 prompt tokens of 5 requests (173 GFLOP) 419 -> 208; 1 x 2048 tokens 218 ->
-// 127; 8 x 64 tokens at 4096 keys 170 -> 100; 512 at 16K keys 264 (1089 TFLOP/s).
+// 123; 8 x 64 tokens at 4096 keys 170 -> 92; 512 at 16K keys 263 (1093 TFLOP/s).
 // Keys go through LDS in sub-tiles of 32, a ring of three buffers filled by
 // direct loads a step ahead, one barrier per step.  Each wave computes the
 // cache slots of the keys it loads two steps ahead from the unit's block ids,

@@ -2924,7 +2924,7 @@ void mla_attn_kernel(MlaArgs a) {
 // sub-tile v - 1, which do not depend on each other, and the softmax of v runs
 // between the MFMAs of PV.  16 heads, us per call with the merge, before -> now:
 // 2921 prompt tokens of 5 requests (173 GFLOP) 419 -> 208; 1 x 2048 tokens 218 ->
-// 123; 8 x 64 tokens at 4096 keys 170 -> 92; 512 at 16K keys 263 (1093 TFLOP/s).
+// 126; 8 x 64 tokens at 4096 keys 170 -> 96; 512 at 16K keys 263 (1093 TFLOP/s).
 // Keys go through LDS in sub-tiles of 32, a ring of three buffers filled by
 // direct loads a step ahead, one barrier per step.  Each wave computes the
 // cache slots of the keys it loads two steps ahead from the unit's block ids,
